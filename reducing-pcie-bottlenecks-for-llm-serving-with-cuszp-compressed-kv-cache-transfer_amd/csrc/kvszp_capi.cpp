@@ -466,18 +466,20 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
     }
     if (job != batch) return fail(KVSZP_EINVAL, "group sizes do not cover the batch");
     const std::vector<Chunk> chunks = split_chunks(specs);
-    uint64_t max_tiles = 0;
+    uint64_t max_tiles = 0, minmax_words = 0;
     for (const Chunk& ch : chunks) {
         if (ch.tiles == 0 || ch.tiles > kMaxTiles)
             return fail(KVSZP_EINVAL, "batch too large for one launch");
         max_tiles = std::max(max_tiles, ch.tiles);
+        minmax_words = std::max(minmax_words, batch * minmax_stride(minmax_shards(
+                                    ch.tiles, ch.max_tiles_per_job, batch, UINT64_MAX)));
     }
 
     const bool relative = c->config.use_relative_error != 0 && !bounds_given;
     // Workspaces.
     if ((rc = ensure(c->tile_state, max_tiles * 8, true, stream)) ||
         (rc = ensure(c->tile_minmax, max_tiles * 8, true, stream)) ||
-        (rc = ensure(c->job_minmax, batch * 16, true, stream)) ||
+        (rc = ensure(c->job_minmax, minmax_words * 8, true, stream)) ||
         (rc = ensure(c->job_flags, batch * 4, true, stream)) ||
         (rc = ensure_host_results(c, batch * 12)))
         return rc;
@@ -520,6 +522,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         CompressParams p;
         std::memset(&p, 0, sizeof(p));
         p.num_groups = fill_groups(p.groups, specs, ch, chunk_first_job[k]);
+        p.minmax_shards = minmax_shards(ch.tiles, ch.max_tiles_per_job, batch, UINT64_MAX);
         int bound_mode = kBoundAbsolute;
         if (relative)
             bound_mode = (!safe && !f32 && ch.max_tiles_per_job <= c->fused_tile_limit)
@@ -554,6 +557,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
                 std::memcpy(m.inline_jobs, jobs.data(), batch * sizeof(CompressJob));
             }
             m.job_minmax = reinterpret_cast<unsigned long long*>(c->job_minmax.ptr);
+            m.minmax_shards = p.minmax_shards;
             m.error = error_word(c);
             m.error_marker = error_marker(c);
             m.host_ctl = c->host_ctl;
@@ -1134,6 +1138,8 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
     g.header_bytes = header_bytes_of(n);
     set_group_divisors(g);
     p.num_groups = 1;
+    p.minmax_shards = minmax_shards((uint64_t)tiles_per_job * batch, tiles_per_job, batch,
+                                    2ull * kNoAllocMaxJobs);
     // After a recent give-up, the schedule that needs no residency at once.
     const bool schedule_safe = c->safe_left > 0;
     if (schedule_safe) {
@@ -1158,6 +1164,7 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
             std::memcpy(m.inline_jobs, c->noalloc_stage, batch * sizeof(CompressJob));
         }
         m.job_minmax = words + kScratchJobMinMax / 8;
+        m.minmax_shards = p.minmax_shards;
         m.error = error_word(c);
         m.error_marker = error_marker(c);
         m.host_ctl = c->host_ctl;
@@ -1227,6 +1234,7 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
                 std::memcpy(m.inline_jobs, c->noalloc_stage, batch * sizeof(CompressJob));
             }
             m.job_minmax = words + kScratchJobMinMax / 8;
+            m.minmax_shards = p.minmax_shards;
             m.error = error_word(c);
             m.error_marker = error_marker(c);
             m.host_ctl = c->host_ctl;

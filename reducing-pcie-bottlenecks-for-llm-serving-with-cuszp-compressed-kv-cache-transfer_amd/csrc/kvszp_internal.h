@@ -101,7 +101,8 @@ struct CompressParams {
     const CompressJob* jobs;
     unsigned long long* tile_state;   // look-back words, one per tile
     unsigned long long* tile_minmax;  // fused min/max words, one per tile
-    const unsigned long long* job_minmax;  // pre-pass words, two per job
+    const unsigned long long* job_minmax;  // pre-pass words (minmax_stride per job)
+    uint32_t minmax_shards;
     uint32_t* host_sizes;             // out (pinned host): stream bytes per job
     float* host_bounds;               // out (pinned host): absolute bound per job
     uint32_t* host_redo;              // out (pinned host): seq = encode the job again
@@ -138,15 +139,18 @@ struct CompressParams {
 
 struct MinMaxParams {
     const CompressJob* jobs;
-    unsigned long long* job_minmax;   // two words per job: max key, ~min key
+    unsigned long long* job_minmax;   // per job and shard: max key, ~min key
+    uint32_t minmax_shards;
     uint32_t* error;
     uint32_t* error_marker;
     uint32_t* host_ctl;
     uint32_t seq;
     uint32_t epoch;
+    uint32_t total_tiles;
+    uint32_t tiles_per_wg;            // consecutive tiles of one workgroup
     int num_groups;
     int input_f32;                    // fp32 pages: 32-bit keys, NaN marked
-    Group groups[kMaxGroups];         // first_tile is the first chunk
+    Group groups[kMaxGroups];
     uint32_t num_jobs;                // job records in the table (jobs or inline_jobs)
     int jobs_inline;                  // 1: the jobs are inline_jobs, not *jobs
     CompressJob inline_jobs[kInlineJobs];
@@ -242,8 +246,9 @@ hipError_t launch_compress_pipelined(const CompressParams& p, uint32_t grid,
                                      hipStream_t stream, hipEvent_t start,
                                      hipEvent_t stop, const void* table = nullptr,
                                      size_t table_bytes = 0);
-hipError_t launch_minmax(const MinMaxParams& p, uint32_t grid,
-                         hipStream_t stream, hipEvent_t start);
+// Pre-pass over `tiles` tiles; fills in p.total_tiles and p.tiles_per_wg.
+hipError_t launch_minmax(MinMaxParams p, uint32_t tiles, hipStream_t stream,
+                         hipEvent_t start);
 hipError_t launch_decompress(const DecompressParams& p, hipStream_t stream,
                              hipEvent_t start, hipEvent_t stop);
 // Persistent decoder: `grid` workgroups each decode a run of consecutive

@@ -49,6 +49,8 @@ typedef __attribute__((address_space(1))) uint32_t g_u32;
 typedef __attribute__((address_space(1))) u32x4 g_u32x4;
 typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
 typedef __attribute__((address_space(1))) u32x4_a4 g_u32x4_a4;
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef __attribute__((address_space(1))) u32x4_a2 g_u32x4_a2;
 
 template <typename T>
 __device__ __forceinline__ __attribute__((address_space(1))) T* to_global(T* p) {
@@ -410,11 +412,13 @@ __device__ __forceinline__ LayerCursor layer_cursor(
 }
 
 // Loads the 32 BF16 values of a block as 16 packed pairs; elements at or
-// past `count` are loaded as 0 (the caller masks them anyway).
+// past `count` are loaded as 0 (the caller masks them anyway).  A whole block
+// inside one layer is four 16-byte loads at any 2-byte address (gfx950 takes
+// them unaligned); as 32 loads of 2 bytes each, a 32 Mi-value segment's
+// pre-pass ran at 0.5 TB/s.
 __device__ __forceinline__ void load_block(
     const Group& g, const uint16_t* in, uint64_t tile_first_elem,
-    uint32_t elem_in_tile, uint32_t count, bool aligned16, uint32_t* d,
-    uint32_t* bad) {
+    uint32_t elem_in_tile, uint32_t count, uint32_t* d, uint32_t* bad) {
     const uint64_t e0 = tile_first_elem + elem_in_tile;
     uint64_t src = e0;
     bool contiguous = true;
@@ -423,8 +427,8 @@ __device__ __forceinline__ void load_block(
         src = c.src_index;
         contiguous = c.contiguous;
     }
-    if (count == kBlockElems && contiguous && aligned16) {
-        const g_u32x4* p = (const g_u32x4*)to_global(in + src);
+    if (count == kBlockElems && contiguous) {
+        const g_u32x4_a2* p = (const g_u32x4_a2*)to_global(in + src);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const u32x4 v = p[i];
@@ -499,17 +503,16 @@ __device__ __forceinline__ void load_block_wave(
         wave_load_blocks(in + src0, lds_wave, d);
         return;
     }
-    load_block(g, in, tile_first_elem, elem_in_tile, count, aligned16, d, bad);
+    load_block(g, in, tile_first_elem, elem_in_tile, count, d, bad);
 }
 
 // The 32 fp32 values of a block starting at element e0 of a contiguous page
 // (values at or past `count` read as 0): eight 16-byte loads when the block
-// is whole and the page 16-byte aligned, else one value at a time.
+// is whole, else one value at a time.
 __device__ __forceinline__ void load_block_f32(const float* in, uint64_t e0,
-                                               uint32_t count, bool aligned16,
-                                               uint32_t* d) {
-    if (count == kBlockElems && aligned16) {
-        const g_u32x4* p = (const g_u32x4*)to_global(in + e0);
+                                               uint32_t count, uint32_t* d) {
+    if (count == kBlockElems) {
+        const g_u32x4_a4* p = (const g_u32x4_a4*)to_global(in + e0);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const u32x4 v = p[i];
@@ -827,6 +830,21 @@ __device__ __forceinline__ void build_rows_hi(const uint32_t* d, uint32_t count,
 
 // ---- encoder ---------------------------------------------------------------
 
+// A job's pre-pass result (minmax_kernel): the largest max key and inverted
+// min key over its shards, on every lane.  False when no shard was written.
+__device__ __forceinline__ bool prepass_words(const CompressParams& p, uint32_t job,
+                                              uint32_t& wmax, uint32_t& wmin) {
+    const uint32_t lane = __lane_id();
+    const unsigned long long* w =
+        p.job_minmax + (size_t)job * minmax_stride(p.minmax_shards) +
+        (lane < p.minmax_shards ? lane : 0u) * kMinMaxShardWords;
+    const unsigned long long a = w[0], b = w[1];
+    const bool written = (uint32_t)(a >> 32) == p.epoch && (uint32_t)(b >> 32) == p.epoch;
+    wmax = wave_max(written ? (uint32_t)a : 0u);
+    wmin = wave_max(written ? (uint32_t)b : 0u);
+    return __ballot(written) != 0ull;
+}
+
 // kIn = 0: BF16 pages (any bound mode, layer maps); kIn = 1: contiguous
 // fp32 pages (absolute or pre-pass bound), the single-page fp32 API.
 template <int kQuant, int kIn>
@@ -869,8 +887,7 @@ __global__ __launch_bounds__(kThreads) void compress_kernel(CompressParams p) {
     uint32_t bad = 0;
     uint32_t d[kIn ? kBlockElems : kBlockElems / 2];
     if constexpr (kIn)
-        load_block_f32(reinterpret_cast<const float*>(J.in), e0, count,
-                       p.aligned16 != 0, d);
+        load_block_f32(reinterpret_cast<const float*>(J.in), e0, count, d);
     else
         load_block_wave(g, J.in, tile_first, (uint32_t)tid * kBlockElems, count,
                         p.aligned16 != 0, d, &bad, &s_stage[wave][0]);
@@ -878,11 +895,9 @@ __global__ __launch_bounds__(kThreads) void compress_kernel(CompressParams p) {
     float eb = J.eps;
     if constexpr (kIn) {
         if (p.bound_mode != kBoundAbsolute) {  // pre-pass words (32-bit keys)
-            const unsigned long long wmax = p.job_minmax[2 * job];
-            const unsigned long long wmin = p.job_minmax[2 * job + 1];
-            if ((uint32_t)(wmax >> 32) != p.epoch || (uint32_t)(wmin >> 32) != p.epoch)
-                bad |= 2;
-            eb = relative_bound_f32(J.eps, 0xFFFFFFFFu - (uint32_t)wmin, (uint32_t)wmax);
+            uint32_t wmax, wmin;
+            if (!prepass_words(p, job, wmax, wmin)) bad |= 2;
+            eb = relative_bound_f32(J.eps, 0xFFFFFFFFu - wmin, wmax);
         }
     } else if (p.bound_mode != kBoundAbsolute) {
         uint32_t kmin, kmax;
@@ -944,13 +959,10 @@ __global__ __launch_bounds__(kThreads) void compress_kernel(CompressParams p) {
                 kmax = s_max[w] > kmax ? s_max[w] : kmax;
             }
         } else {
-            const unsigned long long wmax = p.job_minmax[2 * job];
-            const unsigned long long wmin = p.job_minmax[2 * job + 1];
-            if ((uint32_t)(wmax >> 32) != p.epoch ||
-                (uint32_t)(wmin >> 32) != p.epoch)
-                bad |= 2;  // reported as a spin error below
-            kmax = (uint32_t)wmax & 0xFFFFu;
-            kmin = 0xFFFFu - ((uint32_t)wmin & 0xFFFFu);
+            uint32_t wmax, wmin;
+            if (!prepass_words(p, job, wmax, wmin)) bad |= 2;  // reported as a spin error below
+            kmax = wmax;
+            kmin = 0xFFFFu - wmin;
         }
         eb = relative_bound(J.eps, kmin, kmax);
     }
@@ -1020,11 +1032,9 @@ __global__ __launch_bounds__(kThreads) void compress_kernel(CompressParams p) {
         // Rare, so the block is re-read instead of kept in registers.
         uint32_t bad2 = 0;
         if constexpr (kIn)
-            load_block_f32(reinterpret_cast<const float*>(J.in), e0, count,
-                           p.aligned16 != 0, d);
+            load_block_f32(reinterpret_cast<const float*>(J.in), e0, count, d);
         else
-            load_block(g, J.in, tile_first, (uint32_t)tid * kBlockElems, count,
-                       p.aligned16 != 0, d, &bad2);
+            load_block(g, J.in, tile_first, (uint32_t)tid * kBlockElems, count, d, &bad2);
         if (count == kBlockElems)
             build_rows_hi<kQuant, true, kIn>(d, count, recip, P);
         else
@@ -1146,14 +1156,13 @@ __global__ __launch_bounds__(kThreads) void compress_lorenzo_kernel(CompressPara
         b < nb ? (uint32_t)(n - e0 < kBlockElems ? n - e0 : kBlockElems) : 0u;
 
     uint32_t d[kBlockElems];
-    load_block_f32(reinterpret_cast<const float*>(J.in), e0, count, p.aligned16 != 0, d);
+    load_block_f32(reinterpret_cast<const float*>(J.in), e0, count, d);
     float eb = J.eps;
     uint32_t bad = 0;
     if (p.bound_mode != kBoundAbsolute) {  // pre-pass words (32-bit keys)
-        const unsigned long long wmax = p.job_minmax[2 * job];
-        const unsigned long long wmin = p.job_minmax[2 * job + 1];
-        if ((uint32_t)(wmax >> 32) != p.epoch || (uint32_t)(wmin >> 32) != p.epoch) bad = 1;
-        eb = relative_bound_f32(J.eps, 0xFFFFFFFFu - (uint32_t)wmin, (uint32_t)wmax);
+        uint32_t wmax, wmin;
+        if (!prepass_words(p, job, wmax, wmin)) bad = 1;
+        eb = relative_bound_f32(J.eps, 0xFFFFFFFFu - wmin, wmax);
     }
     const float recip = 0.5f / eb;  // IEEE division, as in fixed mode
 
@@ -2181,70 +2190,164 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void compress_persistent_argtable_ker
 
 // ---- relative-bound pre-pass (jobs too long for the fused exchange) -------
 
-// kIn = 0: BF16 pages, 16-bit keys, NaN ignored (cu:78-79).  kIn = 1:
-// contiguous fp32 pages, 32-bit keys, a NaN marks the max word (at::aminmax
-// propagates NaN, cuszp_wrapper.cpp:253).
+// Order keys of the 32 fp32 values in d[], as minmax_kernel<1> keeps them: the
+// smallest non-NaN key, and the largest key with kKey32Nan for a NaN.  Read
+// as signed numbers, the patterns with the sign bit clear order by value and
+// lie above all others; read as unsigned numbers, those with the sign bit set
+// lie above all others and order by magnitude (see block_keys): two maxima
+// over the raw words serve a set that holds both signs and no NaN.
+__device__ __forceinline__ void keys32_minmax(const uint32_t* d, uint32_t& kmin,
+                                              uint32_t& kmax) {
+    int32_t smax = INT32_MIN;
+    uint32_t umax = 0;
+#pragma unroll
+    for (int v = 0; v < kBlockElems; ++v) {
+        smax = max(smax, (int32_t)d[v]);
+        umax = max(umax, d[v]);
+    }
+    if (smax >= 0 && smax <= 0x7F800000 && umax >= 0x80000000u && umax <= 0xFF800000u) {
+        kmin = ~umax;
+        kmax = (uint32_t)smax | 0x80000000u;
+        return;
+    }
+    kmin = 0xFFFFFFFFu;
+    kmax = 0u;
+#pragma unroll
+    for (int v = 0; v < kBlockElems; ++v) {
+        const float x = __uint_as_float(d[v]);
+        const uint32_t k = x != x ? kKey32Nan : key32(x);
+        kmax = max(kmax, k);
+        if (x == x) kmin = min(kmin, k);
+    }
+}
+
+// First of the 2048 values of wave `wave` of a tile of a BF16 page when they
+// are all there and lie one behind the other (any 2-byte address); nullptr
+// otherwise (each lane then finds its own block).  Wave-uniform.
+__device__ __forceinline__ const uint16_t* whole_run(const Group& g, const uint16_t* in,
+                                                     uint32_t tile, int wave) {
+    constexpr uint32_t kRun = 64u * kBlockElems;
+    const uint32_t E = tile * (uint32_t)kTileElems + (uint32_t)wave * kRun;
+    if ((uint64_t)E + kRun > g.n) return nullptr;
+    if (g.layers == nullptr) return in + E;
+    const uint32_t epl = (uint32_t)g.elements_per_layer;
+    const uint32_t pre = divide(E, g.prefix_div);
+    const uint32_t within = E - pre * ((uint32_t)g.selected_layers * epl);
+    const uint32_t layer = divide(within, g.layer_div);
+    const uint32_t inner = within - layer * epl;
+    if (inner + kRun > epl) return nullptr;
+    const int64_t l = load_const(g.layers, layer);
+    if (l < 0 || (uint64_t)l >= g.source_layers) return nullptr;
+    return in + ((uint64_t)pre * g.source_layers + (uint64_t)l) * epl + inner;
+}
+
+// Min/max over every job's values.  kIn = 0: BF16 pages, 16-bit keys, NaN
+// ignored (cu:78-79).  kIn = 1: contiguous fp32 pages, 32-bit keys, a NaN
+// marks the max word (at::aminmax propagates NaN, cuszp_wrapper.cpp:253).
+//
+// Bound by memory: each value is read once.  A minimum does not care which
+// lane holds which value, so a wave whose 2048 values lie one behind the other
+// reads them as 1 KiB per instruction, at whatever address they start; only
+// waves at the end of a segment, or across layers, go block by block.  A
+// workgroup takes `tiles_per_wg` consecutive tiles and publishes once per job
+// it met.  Atomics to one cache line take about 11 ns each, one after the
+// other: 2048 workgroups publishing to one job's pair of words held a 134 MB
+// pass at 43 us where the same reads with no publishing take 27.  A job of
+// many workgroups therefore has up to 32 pairs, each on a line of its own
+// (minmax_shards, kvszp_plan.h), which the encoder's waves read at once.
 template <int kIn>
 __global__ __launch_bounds__(kThreads) void minmax_kernel(MinMaxParams p) {
-    __shared__ uint32_t s_min[kThreads / 64];
-    __shared__ uint32_t s_max[kThreads / 64];
+    __shared__ uint32_t s_min[2][kThreads / 64];
+    __shared__ uint32_t s_max[2][kThreads / 64];
+    constexpr uint32_t kEmpty = kIn ? 0xFFFFFFFFu : kKeyEmptyMin;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     publish_seq(p.host_ctl, p.seq);
-    const uint32_t t = blockIdx.x;
-    const Group& g = p.groups[find_group(p.groups, p.num_groups, t)];
-    const uint32_t local = t - g.first_tile;
-    const uint32_t job_in_group = local / g.tiles_per_job;
-    const uint32_t tile = local - job_in_group * g.tiles_per_job;
-    const uint32_t job = g.first_job + job_in_group;
-    const CompressJob J = job_at(p, job);
-    const uint64_t n = g.n;
-    const uint32_t nb = (uint32_t)((n + kBlockElems - 1) / kBlockElems);
-    const uint32_t b = tile * kTileBlocks + tid;
-    const uint64_t e0 = (uint64_t)b * kBlockElems;
-    const uint32_t count =
-        b < nb ? (uint32_t)(n - e0 < kBlockElems ? n - e0 : kBlockElems) : 0u;
-    uint32_t bad = 0;
-    uint32_t kmin, kmax;
-    if constexpr (kIn) {
-        uint32_t d[kBlockElems];
-        load_block_f32(reinterpret_cast<const float*>(J.in), e0, count,
-                       ((uintptr_t)J.in & 15u) == 0, d);
-        kmin = 0xFFFFFFFFu;
-        kmax = 0u;
-        for (uint32_t v = 0; v < count; ++v) {
-            const float x = __uint_as_float(d[v]);
-            const uint32_t k = x != x ? kKey32Nan : key32(x);
-            kmax = k > kmax ? k : kmax;
-            if (x == x) kmin = k < kmin ? k : kmin;
-        }
-    } else {
-        uint32_t d[16];
-        load_block(g, J.in, (uint64_t)tile * kTileElems, (uint32_t)tid * kBlockElems,
-                   count, false, d, &bad);
-        block_key_minmax(d, count, kmin, kmax);
-    }
-    kmin = wave_min(kmin);
-    kmax = wave_max(kmax);
-    if (lane == 0) {
-        s_min[wave] = kmin;
-        s_max[wave] = kmax;
-    }
-    __syncthreads();
-    if (tid == 0) {
+    uint32_t t = blockIdx.x * p.tiles_per_wg;
+    const uint32_t end = min(t + p.tiles_per_wg, p.total_tiles);
+    uint32_t bad = 0, lo = kEmpty, hi = 0;
+    for (int flushes = 0; t < end;) {
+        const Group& g = p.groups[find_group(p.groups, p.num_groups, t)];
+        const uint32_t local = t - g.first_tile;
+        const uint32_t job_in_group =
+            __builtin_amdgcn_readfirstlane(divide(local, g.tiles_per_job_div));
+        const uint32_t tile = local - job_in_group * g.tiles_per_job;
+        const uint32_t job = g.first_job + job_in_group;
+        const CompressJob J = job_at(p, job);
+        const uint64_t e0 = ((uint64_t)tile * kTileBlocks + tid) * kBlockElems;
+        const uint32_t count =
+            e0 < g.n ? (uint32_t)(g.n - e0 < kBlockElems ? g.n - e0 : kBlockElems) : 0u;
+        uint32_t kmin = kEmpty, kmax = 0;
+        if constexpr (kIn) {
+            uint32_t d[kBlockElems];
+            const uint64_t E = (uint64_t)tile * kTileElems + (uint32_t)wave * 64u * kBlockElems;
+            const float* in = reinterpret_cast<const float*>(J.in);
+            if (E + 64u * kBlockElems <= g.n) {
+                const g_u32* src = to_global(reinterpret_cast<const uint32_t*>(in + E)) + 4 * lane;
 #pragma unroll
-        for (int w = 1; w < kThreads / 64; ++w) {
-            kmin = s_min[w] < kmin ? s_min[w] : kmin;
-            kmax = s_max[w] > kmax ? s_max[w] : kmax;
+                for (int i = 0; i < 8; ++i) {
+                    const u32x4 v = *(const g_u32x4_a4*)(src + 256 * i);
+                    d[4 * i + 0] = v.x;
+                    d[4 * i + 1] = v.y;
+                    d[4 * i + 2] = v.z;
+                    d[4 * i + 3] = v.w;
+                }
+                keys32_minmax(d, kmin, kmax);
+            } else if (count) {
+                // a block's missing values repeat its first one
+                const g_u32* src = to_global(reinterpret_cast<const uint32_t*>(in + e0));
+#pragma unroll
+                for (int v = 0; v < kBlockElems; ++v)
+                    d[v] = src[(uint32_t)v < count ? v : 0];
+                keys32_minmax(d, kmin, kmax);
+            }
+        } else {
+            uint32_t d[16];
+            const uint16_t* run = whole_run(g, J.in, tile, wave);
+            if (run != nullptr) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const u32x4 v = *(const g_u32x4_a2*)to_global(run + 512 * i + 8 * lane);
+                    d[4 * i + 0] = v.x;
+                    d[4 * i + 1] = v.y;
+                    d[4 * i + 2] = v.z;
+                    d[4 * i + 3] = v.w;
+                }
+                block_key_minmax(d, kBlockElems, kmin, kmax);
+            } else {
+                load_block(g, J.in, (uint64_t)tile * kTileElems, (uint32_t)tid * kBlockElems,
+                           count, d, &bad);
+                block_key_minmax(d, count, kmin, kmax);
+            }
         }
-        const unsigned long long tag = (unsigned long long)p.epoch << 32;
-        __hip_atomic_fetch_max(&p.job_minmax[2 * job], tag | kmax,
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t key_max = kIn ? 0xFFFFFFFFu : 0xFFFFu;
-        __hip_atomic_fetch_max(&p.job_minmax[2 * job + 1],
-                               tag | (key_max - kmin), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+        lo = min(lo, kmin);
+        hi = max(hi, kmax);
+        ++t;
+        if (t < end && tile + 1 < g.tiles_per_job) continue;  // the same job goes on
+        const uint32_t wlo = wave_min(lo), whi = wave_max(hi);
+        // by parity: the words of the flush before last have been read
+        uint32_t* mn = s_min[flushes & 1];
+        uint32_t* mx = s_max[flushes & 1];
+        if (lane == 0) {
+            mn[wave] = wlo;
+            mx[wave] = whi;
+        }
+        __syncthreads();
+        if (tid < 2) {  // thread 0: the max word, thread 1: the (inverted) min word
+            uint32_t v = 0;
+#pragma unroll
+            for (int w = 0; w < kThreads / 64; ++w)
+                v = max(v, tid == 0 ? mx[w] : kEmpty - mn[w]);
+            const uint32_t shard = (tile / p.tiles_per_wg) & (p.minmax_shards - 1u);
+            __hip_atomic_fetch_max(&p.job_minmax[(size_t)job * minmax_stride(p.minmax_shards) +
+                                                 shard * kMinMaxShardWords + tid],
+                                   ((unsigned long long)p.epoch << 32) | v, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        }
+        ++flushes;
+        lo = kEmpty;
+        hi = 0;
     }
     if (bad) flag_error(p.error, p.error_marker, kErrLayerIndex);
 }
@@ -3183,9 +3286,13 @@ hipError_t launch_compress_pipelined(const CompressParams& p, uint32_t grid,
     return hipGetLastError();
 }
 
-hipError_t launch_minmax(const MinMaxParams& p, uint32_t grid,
-                         hipStream_t stream, hipEvent_t start) {
-    if (!tile_plan_ok(p.groups, p.num_groups, grid, grid, false, readable_jobs(p)))  // a workgroup per tile
+hipError_t launch_minmax(MinMaxParams p, uint32_t tiles, hipStream_t stream,
+                         hipEvent_t start) {
+    // Enough workgroups to fill the chip several times over, then more tiles each.
+    p.total_tiles = tiles;
+    p.tiles_per_wg = minmax_tiles_per_wg(tiles);
+    const uint32_t grid = (tiles + p.tiles_per_wg - 1) / p.tiles_per_wg;
+    if (!tile_plan_ok(p.groups, p.num_groups, tiles, grid, false, readable_jobs(p)))
         return hipErrorInvalidValue;
     if (p.input_f32)
         launch(minmax_kernel<1>, grid, stream, start, nullptr, p);

@@ -138,6 +138,40 @@ KVSZP_PLAN_FN uint32_t weighted_run_start(const Group* groups, int num_groups,
     return first + (i < (double)tiles ? (uint32_t)i : tiles);
 }
 
+// ---- the relative-bound pre-pass ---------------------------------------------
+
+// Its workgroups take 1 to kMinMaxTilesPerWg consecutive tiles each, as many
+// as leave kMinMaxWorkgroups workgroups (8 on each of 256 compute units).
+constexpr uint32_t kMinMaxWorkgroups = 2048;
+constexpr uint32_t kMinMaxTilesPerWg = 4;
+// A job's words are `shards` pairs (max key, inverted min key), one 64-byte
+// line apart, so that the atomics of a job's workgroups spread over lines; a
+// job with one shard takes just its pair.
+constexpr uint32_t kMinMaxShardWords = 8;
+constexpr uint32_t kMinMaxShards = 32;
+
+KVSZP_PLAN_FN uint32_t minmax_tiles_per_wg(uint64_t tiles) {
+    const uint64_t per = tiles / kMinMaxWorkgroups;
+    return per < 1 ? 1u : per < kMinMaxTilesPerWg ? (uint32_t)per : kMinMaxTilesPerWg;
+}
+
+KVSZP_PLAN_FN uint32_t minmax_stride(uint32_t shards) {
+    return shards > 1 ? shards * kMinMaxShardWords : 2u;
+}
+
+// Shards of each job of a launch of `tiles` tiles whose longest job has
+// `tiles_per_job`: a power of two, one per 16 workgroups of that job (16
+// atomics on a line take 0.2 us), as far as `words` words hold `jobs` jobs.
+inline uint32_t minmax_shards(uint64_t tiles, uint32_t tiles_per_job, uint64_t jobs,
+                              uint64_t words) {
+    const uint32_t wgs = tiles_per_job / minmax_tiles_per_wg(tiles);
+    uint32_t shards = 1;
+    while (shards < kMinMaxShards && 16u * shards < wgs &&
+           jobs * minmax_stride(2 * shards) <= words)
+        shards *= 2;
+    return shards;
+}
+
 // ---- host: building and checking a plan ------------------------------------
 
 // Header bytes of a segment of n values: one rate byte per block, for whole
