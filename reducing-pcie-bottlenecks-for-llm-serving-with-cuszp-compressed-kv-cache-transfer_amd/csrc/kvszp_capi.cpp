@@ -704,7 +704,7 @@ int decompress_groups(kvszp_ctx* c, const void* const* compressed,
                       const std::vector<GroupSpec>& specs, int dst_kind,
                       const std::vector<uint16_t*>& dst_base,
                       const std::vector<uint16_t*>& dest_table, uint64_t dpp,
-                      uint64_t epd, bool aligned16, hipStream_t stream,
+                      uint64_t epd, hipStream_t stream,
                       bool f32 = false, uint32_t grid_cap = 0, int mode = kModeFixed) {
     int rc = use_device(c);
     if (rc) return rc;
@@ -835,11 +835,11 @@ int decompress_groups(kvszp_ctx* c, const void* const* compressed,
         p.total_tiles = (uint32_t)ch.tiles;
         p.dst_kind = dst_kind;
         p.rate0_zero = c->rate0 == KVSZP_RATE0_ZERO ? 1 : 0;
-        p.aligned16 = aligned16 ? 1 : 0;
         p.output_f32 = f32 ? 1 : 0;
         p.mode = f32 ? mode : kModeFixed;
         p.dests_per_page = dpp;
         p.elements_per_dest = epd;
+        p.dest_div = divisor_of((uint32_t)epd);
         const int rec = timing_begin(c, KVSZP_KERNEL_DECOMPRESS);
         hipError_t e;
         if (persistent_for(ch.tiles)) {
@@ -1328,13 +1328,10 @@ int kvszp_decompress_batch_fixed_bf16(kvszp_ctx* c, const void* const* compresse
     std::vector<uint16_t*> base(batch);
     for (size_t i = 0; i < batch; ++i)
         base[i] = reinterpret_cast<uint16_t*>(output) + i * num_elements_per_page;
-    const bool aligned16 =
-        ((uintptr_t)output & 15u) == 0 && (num_elements_per_page % 8) == 0;
     const std::vector<GroupSpec> spec{
         GroupSpec{num_elements_per_page, nullptr, 0, 0, 0, (uint32_t)batch}};
     return decompress_groups(c, compressed, sizes, error_bounds, batch, spec,
-                             kDstLinear, base, {}, 0, 0, aligned16,
-                             (hipStream_t)stream);
+                             kDstLinear, base, {}, 0, 0, (hipStream_t)stream);
 }
 
 int kvszp_decompress_batch_fixed_bf16_scatter(
@@ -1353,12 +1350,10 @@ int kvszp_decompress_batch_fixed_bf16_scatter(
         return fail(KVSZP_EINVAL, "invalid direct-scatter metadata");
     const size_t count = batch * destinations_per_page;
     std::vector<uint16_t*> dests(count);
-    bool aligned16 = true;
     for (size_t i = 0; i < count; ++i) {
         const uintptr_t d = (uintptr_t)destinations[i];
         if (!d || (d & 1u))
             return fail(KVSZP_EINVAL, "invalid BF16 direct-scatter destination %zu", i);
-        if (d & 15u) aligned16 = false;
         dests[i] = reinterpret_cast<uint16_t*>(d);
     }
     const std::vector<GroupSpec> spec{
@@ -1367,13 +1362,11 @@ int kvszp_decompress_batch_fixed_bf16_scatter(
         // One destination per page: straight 16-byte stores into the page
         // (cu:383-386, 566-576).
         return decompress_groups(c, compressed, sizes, error_bounds, batch, spec,
-                                 kDstLinear, dests, {}, 0, 0,
-                                 aligned16 && (num_elements_per_page % 8) == 0,
-                                 (hipStream_t)stream);
+                                 kDstLinear, dests, {}, 0, 0, (hipStream_t)stream);
     }
     return decompress_groups(c, compressed, sizes, error_bounds, batch, spec,
                              kDstMulti, {}, dests, destinations_per_page,
-                             elements_per_destination, false, (hipStream_t)stream);
+                             elements_per_destination, (hipStream_t)stream);
 }
 
 int kvszp_decompress_batch_fixed_bf16_indexed_scatter(
@@ -1402,8 +1395,7 @@ int kvszp_decompress_batch_fixed_bf16_indexed_scatter(
                   layer_indices, selected_layers, source_layers, elements_per_layer,
                   (uint32_t)batch}};
     return decompress_groups(c, compressed, sizes, error_bounds, batch, spec,
-                             kDstIndexed, dests, {}, 0, 0, false,
-                             (hipStream_t)stream);
+                             kDstIndexed, dests, {}, 0, 0, (hipStream_t)stream);
 }
 
 int kvszp_decompress_batch_fixed_bf16_indexed_scatter_groups(
@@ -1445,8 +1437,7 @@ int kvszp_decompress_batch_fixed_bf16_indexed_scatter_groups(
         dests[i] = reinterpret_cast<uint16_t*>(d);
     }
     return decompress_groups(c, compressed, sizes, error_bounds, batch, specs,
-                             kDstIndexed, dests, {}, 0, 0, false,
-                             (hipStream_t)stream);
+                             kDstIndexed, dests, {}, 0, 0, (hipStream_t)stream);
 }
 
 int kvszp_compress_fixed_f32(kvszp_ctx* c, const float* input, size_t num_elements,
@@ -1488,19 +1479,17 @@ static int decompress_f32(kvszp_ctx* c, const void* const* compressed,
         return fail(KVSZP_EINVAL, "null pointer argument");
     std::vector<GroupSpec> specs;
     std::vector<uint16_t*> base(batch);
-    bool aligned16 = true;
     for (size_t i = 0; i < batch; ++i) {
         const uintptr_t d = (uintptr_t)outputs[i];
         if (!d || (d & 3u)) return fail(KVSZP_EINVAL, "invalid fp32 output %zu", i);
         if (num_elements[i] == 0) return fail(KVSZP_EINVAL, "empty output %zu", i);
-        if (d & 15u) aligned16 = false;
         base[i] = reinterpret_cast<uint16_t*>(d);
         if (specs.empty() || specs.back().n != num_elements[i])
             specs.push_back(GroupSpec{num_elements[i], nullptr, 0, 0, 0, 0});
         specs.back().jobs += 1;
     }
     return decompress_groups(c, compressed, sizes, error_bounds, batch, specs,
-                             kDstLinear, base, {}, 0, 0, aligned16, stream, true, 0,
+                             kDstLinear, base, {}, 0, 0, stream, true, 0,
                              any_mode ? c->config.encoding_mode : kModeFixed);
 }
 
@@ -1683,7 +1672,7 @@ int kvszp_decompress_batch_fixed_bf16_indexed_scatter_groups_packed(
         grid_cap = kLinkDecodeGrid;
     }
     return decompress_groups(c, streams.data(), sizes, error_bounds, batch, specs,
-                             kDstIndexed, dests, {}, 0, 0, false, (hipStream_t)stream,
+                             kDstIndexed, dests, {}, 0, 0, (hipStream_t)stream,
                              false, grid_cap);
 }
 

@@ -171,11 +171,11 @@ struct DecompressParams {
     int num_groups;
     int dst_kind;
     int rate0_zero;                   // 1: write +0.0 for rate-0 blocks
-    int aligned16;                    // every destination base 16B aligned
     int output_f32;                   // write fp32 values (kDstLinear only)
     int mode;                         // fp32 streams: kModeFixed/Plain/Outlier
     uint64_t dests_per_page;
     uint64_t elements_per_dest;
+    Divisor dest_div;                 // by elements_per_dest (kDstMulti)
     // Persistent decoder runs balanced by bytes moved: each tile of group
     // g weighs tile_weight[g] (its BF16 output plus the group's average
     // payload per tile), weight_before[g] is the weight of the tiles before
