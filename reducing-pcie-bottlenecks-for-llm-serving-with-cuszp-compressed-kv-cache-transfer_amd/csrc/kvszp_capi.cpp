@@ -422,7 +422,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
 
     const uintptr_t elem_align = f32 ? 3u : 1u;
     std::vector<CompressJob> jobs(batch);
-    bool aligned16 = true;
+    bool aligned16 = true, negative_bound = false;
     size_t job = 0;
     for (size_t gi = 0; gi < specs.size(); ++gi) {
         const GroupSpec& s = specs[gi];
@@ -461,6 +461,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
             jobs[job].in = reinterpret_cast<const uint16_t*>(in);
             jobs[job].out = reinterpret_cast<uint8_t*>(out);
             jobs[job].eps = e;
+            negative_bound |= e < 0.0f;
             jobs[job].reserved = 0;
         }
     }
@@ -527,12 +528,10 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         if (relative)
             bound_mode = (!safe && !f32 && ch.max_tiles_per_job <= c->fused_tile_limit)
                              ? kBoundFused : kBoundPrepass;
-        // Persistent encoder (whole, aligned, single-layer blocks only); its
-        // waits are cycle-free while a job's tiles number at most the grid
-        // (half of it here, for margin) and all its workgroups are resident.
-        const bool persistent = !safe && !f32 && bound_mode != kBoundPrepass &&
-                                c->pipelined_grid != 0 && ch.whole_blocks && aligned16 &&
-                                ch.max_tiles_per_job <= c->pipelined_grid / 2;
+        const bool persistent =
+            !safe && !f32 && bound_mode != kBoundPrepass &&
+            persistent_encoder_takes(c->pipelined_grid, ch.one_layer_blocks,
+                                     ch.max_tiles_per_job, negative_bound);
         const bool use_arg = persistent && arg_table;
         if (!use_arg) {
             const int r = need_table();
@@ -1094,7 +1093,7 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
     rc = use_device(c);
     if (rc) return rc;
     const uint64_t need = std::max<uint64_t>(8ull * n, header_bytes_of(n) + 128ull * ((n + 31) / 32));
-    bool aligned16 = true;
+    bool aligned16 = true, negative_bound = false;
     for (size_t i = 0; i < batch; ++i) {
         const uintptr_t in = (uintptr_t)inputs[i], out = (uintptr_t)outputs[i];
         if (!in || !out) return fail(KVSZP_EINVAL, "null page pointer %zu", i);
@@ -1110,6 +1109,7 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
         j.eps = (eps_overrides && eps_overrides[i] > 0.0f) ? eps_overrides[i]
                                                           : c->config.error_bound;
         j.reserved = 0;
+        negative_bound |= j.eps < 0.0f;
     }
     // The previous call on this context waited for its kernels, so the
     // staging records are free; the copy goes into the scratch job table.
@@ -1126,7 +1126,6 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
     if ((rc = scratch_epoch(c, stream, &epoch))) return rc;
 
     const bool relative = c->config.use_relative_error != 0;
-    const bool whole_blocks = (n % kBlockElems) == 0;
     const uint32_t seq = ++c->seq;
     CompressParams p;
     std::memset(&p, 0, sizeof(p));
@@ -1197,9 +1196,9 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
     p.bound_mode = bound_mode;
     p.quantizer = c->quantizer;
     p.aligned16 = aligned16 ? 1 : 0;
-    const bool persistent = !schedule_safe && bound_mode != kBoundPrepass &&
-                            c->pipelined_grid != 0 && whole_blocks && aligned16 &&
-                            tiles_per_job <= c->pipelined_grid / 2;
+    const bool persistent =
+        !schedule_safe && bound_mode != kBoundPrepass &&
+        persistent_encoder_takes(c->pipelined_grid, true, tiles_per_job, negative_bound);
     if (persistent || bound_mode == kBoundFused) {
         p.abort_word = words + kScratchAbort / 8;
         p.wait_ticks = c->wait_ticks;

@@ -1224,9 +1224,9 @@ __global__ __launch_bounds__(kThreads) void compress_lorenzo_kernel(CompressPara
 
 // ---- persistent encoder ----------------------------------------------------
 //
-// For launches whose blocks are all whole, inside one layer and 16-byte
-// aligned (every segment length and layer length a multiple of 32 values,
-// every page 16-byte aligned) -- the shape of KV pages.  Workgroup w encodes
+// For launches whose blocks lie inside one layer each (every layer length a
+// multiple of 32 values; segments without a layer map may have any length and
+// pages any 2-byte address).  Workgroup w encodes
 // tiles w, w + G, w + 2G, ... (G = gridDim.x, at most the number of
 // co-resident workgroups), one 32-value block per thread held in registers
 // together with the block's min/max keys.  Per tile t:
@@ -1287,38 +1287,14 @@ __device__ __forceinline__ TileCtx tile_ctx(const CompressParams& p, uint32_t t,
     return c;
 }
 
-// Whether this thread's block exists (all existing blocks are whole here).
+// Whether this thread's block exists, and whether all its values do (a
+// segment's last block may be cut short; segments hold below 2^29 values).
 __device__ __forceinline__ bool block_exists(const Group& g, uint32_t tile, int tid) {
     return (tile * kTileBlocks + (uint32_t)tid) * kBlockElems < (uint32_t)g.n;
 }
-
-// Source element of this thread's block.  A wave's 64 blocks inside one
-// layer are placed with wave-uniform (scalar) arithmetic and one scalar load
-// of the layer map; otherwise each lane maps its own block.  Element indices
-// of a segment are below 2^29.
-__device__ __forceinline__ uint64_t enc_block_source(const Group& g, uint32_t tile,
-                                                     int wave, int lane, uint32_t* bad) {
-    constexpr uint32_t kRun = 64u * kBlockElems;
-    const uint32_t E = tile * (uint32_t)kTileElems + (uint32_t)wave * kRun;
-    if (g.layers == nullptr) return E + (uint32_t)lane * kBlockElems;
-    const uint32_t epl = (uint32_t)g.elements_per_layer;
-    const uint32_t per_prefix = (uint32_t)g.selected_layers * epl;
-    const uint32_t pre = divide(E, g.prefix_div);
-    const uint32_t within = E - pre * per_prefix;
-    const uint32_t layer = divide(within, g.layer_div);
-    const uint32_t inner = within - layer * epl;
-    if (inner + kRun <= epl) {
-        int64_t l = load_const(g.layers, layer);
-        if (l < 0 || (uint64_t)l >= g.source_layers) {
-            *bad = 1;
-            l = 0;
-        }
-        return ((uint64_t)pre * g.source_layers + (uint64_t)l) * epl + inner +
-               (uint32_t)lane * kBlockElems;
-    }
-    return layer_cursor(g, (uint64_t)tile * kTileElems,
-                        ((uint32_t)wave * 64u + (uint32_t)lane) * kBlockElems, bad)
-        .src_index;
+__device__ __forceinline__ bool block_whole(const Group& g, uint32_t tile, int tid) {
+    return (int32_t)((tile * kTileBlocks + (uint32_t)tid) * kBlockElems) <
+           (int32_t)g.n - (kBlockElems - 1);
 }
 
 // Sixteen zero words, the source of blocks that do not exist: every lane
@@ -1327,32 +1303,20 @@ __device__ __forceinline__ uint64_t enc_block_source(const Group& g, uint32_t ti
 // load, which would tie the persistent encoder's polls to its prefetch.)
 __device__ __attribute__((aligned(16))) uint32_t g_zero_block[kBlockElems / 2];
 
-// This thread's block (zeros when it does not exist, or when `live` is
-// false): four 16-byte loads.  A layer index outside [0, source_layers) is
-// reported at once (the block is then read from layer 0).
-__device__ __forceinline__ void load_block_regs(const CompressParams& p, const TileCtx& c,
-                                                const Group& g, int wave, int lane,
-                                                uint32_t* d, bool live = true) {
-    const bool ex = live && block_exists(g, c.tile, wave * 64 + lane);
-    uint32_t bad = 0;
-    const uint64_t off = ex ? enc_block_source(g, c.tile, wave, lane, &bad) : 0;
-    if (bad) flag_error(p.error, p.error_marker, kErrLayerIndex);
-    const g_u32x4* src = ex ? (const g_u32x4*)to_global(job_of(p, c).in + off)
-                            : (const g_u32x4*)to_global(&g_zero_block[0]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const u32x4 v = src[i];
-        d[4 * i + 0] = v.x;
-        d[4 * i + 1] = v.y;
-        d[4 * i + 2] = v.z;
-        d[4 * i + 3] = v.w;
-    }
-}
+// The kinds of persistent encoder launches.
+enum : int {
+    kEncPlain = 0,  // whole blocks, every wave's run inside one layer
+    // A segment ends inside a block (then there is no layer map).  256 segments
+    // of 100003 values: 28.5 us, one workgroup per tile 41 us.
+    kEncCut = 1,
+    // Layers that are no whole number of runs.  128 blocks of 36 layers of
+    // 6400 values: 57.5 us, with each lane mapping its own block 59.3 us.
+    kEncSplit = 2,
+};
 
-// Source of a tile's blocks for one wave, worked out ahead of the loads: when
-// the wave's 64 blocks are consecutive in memory, `base` is its first block
-// (wave-uniform) and lane l reads base + 32 l; otherwise base is null and
-// each lane maps its own block when loading.
+// Source of a tile's blocks for one wave, worked out ahead of the loads with
+// wave-uniform arithmetic: lane l reads base + 32 l.  A null base means a bad
+// layer index, or a run that crosses into another layer.
 struct WaveSource {
     const uint16_t* base;
 };
@@ -1380,18 +1344,74 @@ __device__ __forceinline__ WaveSource wave_source(const CompressParams& p, const
     return s;
 }
 
-// This thread's block from a WaveSource (zeros when it does not exist, or
-// when `live` is false).
-__device__ __forceinline__ void load_block_from(const CompressParams& p, const TileCtx& c,
-                                                const Group& g, WaveSource s, int wave,
-                                                int lane, uint32_t* d, bool live) {
-    if (s.base == nullptr) {
-        load_block_regs(p, c, g, wave, lane, d, live);
-        return;
+// The same where a run may go on in the next layer of the map: lane l reads
+// base + 32 l, from lane `split` on rest + 32 l.  Null for layers shorter than
+// a run as well, and when either layer index is bad: each lane then maps its
+// own block.
+struct SplitSource {
+    const uint16_t* base;
+    const uint16_t* rest;
+    uint32_t split;
+};
+
+__device__ __forceinline__ SplitSource split_source(const CompressParams& p, const TileCtx& c,
+                                                    const Group& g, int wave) {
+    constexpr uint32_t kRun = 64u * kBlockElems;
+    const uint16_t* in = job_of(p, c).in;
+    const uint32_t E = c.tile * (uint32_t)kTileElems + (uint32_t)wave * kRun;
+    SplitSource s = {in + E, nullptr, 64u};
+    if (g.layers == nullptr) return s;
+    const uint32_t epl = (uint32_t)g.elements_per_layer;
+    const uint32_t sel = (uint32_t)g.selected_layers;
+    const uint32_t pre = divide(E, g.prefix_div);
+    const uint32_t within = E - pre * (sel * epl);
+    const uint32_t layer = divide(within, g.layer_div);
+    const uint32_t inner = within - layer * epl, left = epl - inner;
+    const int64_t l = load_const(g.layers, layer);
+    s.base = epl >= kRun && l >= 0 && (uint64_t)l < g.source_layers
+                 ? in + ((uint64_t)pre * g.source_layers + (uint64_t)l) * epl + inner
+                 : nullptr;
+    if (s.base != nullptr && left < kRun) {
+        const bool wraps = layer + 1u == sel;  // on to the next prefix's first layer
+        const int64_t m = load_const(g.layers, wraps ? 0u : layer + 1u);
+        if (m < 0 || (uint64_t)m >= g.source_layers) s.base = nullptr;
+        s.split = left / kBlockElems;
+        s.rest = in + ((uint64_t)(pre + (wraps ? 1u : 0u)) * g.source_layers + (uint64_t)m) * epl -
+                 left;
     }
-    const bool ex = live && block_exists(g, c.tile, wave * 64 + lane);
-    const g_u32x4* src = ex ? (const g_u32x4*)to_global(s.base + (uint32_t)lane * kBlockElems)
-                            : (const g_u32x4*)to_global(&g_zero_block[0]);
+    return s;
+}
+
+// This thread's block of run `wave` of a tile (zeros when it is not whole, or
+// when `live` is false).  Except for kEncSplit every run lies inside one layer, so
+// that a null base means a bad layer index (reported here).
+template <int kKind>
+__device__ __forceinline__ void load_block_from(const CompressParams& p, const TileCtx& c,
+                                                const Group& g, int wave, int lane,
+                                                uint32_t* d, bool live) {
+    const uint16_t* run;  // this lane's block
+    bool ex = live;
+    if constexpr (kKind == kEncSplit) {
+        const SplitSource s = split_source(p, c, g, wave);
+        if (s.base != nullptr) {
+            run = ((uint32_t)lane >= s.split ? s.rest : s.base) + (uint32_t)lane * kBlockElems;
+        } else {
+            uint32_t bad = 0;
+            run = job_of(p, c).in +
+                  layer_cursor(g, (uint64_t)c.tile * kTileElems,
+                               ((uint32_t)wave * 64u + (uint32_t)lane) * kBlockElems, &bad)
+                      .src_index;
+            if (bad && live) flag_error(p.error, p.error_marker, kErrLayerIndex);
+        }
+    } else {
+        const WaveSource s = wave_source(p, c, g, wave);
+        if (s.base == nullptr && live) flag_error(p.error, p.error_marker, kErrLayerIndex);
+        ex = live && s.base != nullptr;
+        run = s.base + (uint32_t)lane * kBlockElems;
+    }
+    ex = ex && block_whole(g, c.tile, wave * 64 + lane);
+    const g_u32x4_a2* src = ex ? (const g_u32x4_a2*)to_global(run)
+                               : (const g_u32x4_a2*)to_global(&g_zero_block[0]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const u32x4 v = src[i];
@@ -1457,6 +1477,54 @@ __device__ __forceinline__ uint32_t block_keys(const uint32_t* d, bool exists,
 // Keys of -inf (min) and +inf (max), kept as the keys of a block holding a
 // NaN: they mark the block so that its wave takes the exact quantizer.
 constexpr uint32_t kNanRateKeys = (0x007Fu << 16) | 0xFF80u;
+
+// A segment's last block when it is cut short (n a non-multiple of 32; such
+// segments have no layer map): one wave of the tile's two holds it.  Called by
+// a wave after its loads (which read zeros for that block) have arrived, so
+// that the loads stay the same on every path: the wave fetches the values
+// with one load, through LDS, and the block's lane takes the keys of the
+// values there are (the missing ones repeat the first) and the values with
+// zeros for the missing ones, which quantize to 0 while recip is finite.
+__device__ __forceinline__ bool has_cut_block(const Group& g, uint32_t tile, int wave) {
+    const uint32_t first = tile * kTileBlocks + 128u * (uint32_t)wave;
+    const uint32_t last = (uint32_t)g.n / kBlockElems;  // the cut block, if there is one
+    return ((uint32_t)g.n % kBlockElems) != 0u && last >= first && last < first + 128u;
+}
+
+__device__ __forceinline__ void take_cut_block(const Group& g, const uint16_t* in,
+                                               uint32_t tile, int wave, int lane,
+                                               uint16_t* s_cut, uint32_t* d0, uint32_t* d1,
+                                               uint32_t& keys0, uint32_t& keys1,
+                                               uint32_t& nan0, uint32_t& nan1) {
+    const uint32_t last = (uint32_t)g.n / kBlockElems, count = (uint32_t)g.n % kBlockElems;
+    const uint32_t at = last - (tile * kTileBlocks + 128u * (uint32_t)wave);
+    const uint32_t v = (uint32_t)lane & 31u;
+    s_cut[v] = to_global(in)[last * kBlockElems + (v < count ? v : 0u)];
+    __builtin_amdgcn_wave_barrier();
+    __asm__ volatile("" ::: "memory");
+    uint32_t d[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) d[i] = reinterpret_cast<const uint32_t*>(s_cut)[i];
+    __builtin_amdgcn_wave_barrier();
+    __asm__ volatile("" ::: "memory");  // before the words are reused
+    uint32_t nan;
+    const uint32_t keys = block_keys(d, true, nan);
+    const bool mine = (uint32_t)lane == (at & 63u);
+    if (mine && at < 64u) {
+        keys0 = keys;
+        nan0 = nan;
+    }
+    if (mine && at >= 64u) {
+        keys1 = keys;
+        nan1 = nan;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t w = d[i] & (2u * i + 1u < count ? ~0u : 2u * i < count ? 0xFFFFu : 0u);
+        if (mine && at < 64u) d0[i] = w;
+        if (mine && at >= 64u) d1[i] = w;
+    }
+}
 
 // Rate of a block from its keys, for a block whose values all satisfy
 // |x * recip| <= kFastLimit and that holds no NaN: the quantizer is monotone
@@ -1755,7 +1823,12 @@ __device__ __forceinline__ void stage_high_words(const uint32_t* P, uint32_t cou
 // again with the pre-pass schedule (no residency assumption).  Normal waits
 // last microseconds; the bound is hundreds, so the mark costs nothing when
 // the device is not contended.
-template <int kQuant, bool kEarly>
+//
+// kKind: what the launch's blocks need beside the plain loads.  Instantiations
+// of their own: with the other kinds' paths in every launch, those that need
+// neither ran 1-2 % slower (2048 blocks of 458752 values: 668-674 us against
+// 660; without either path, 656-660).
+template <int kQuant, bool kEarly, int kKind>
 __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
     __shared__ uint32_t s_wave[2][kEncWaves];
     __shared__ uint32_t s_min[kEncWaves], s_max[kEncWaves];
@@ -1769,6 +1842,7 @@ __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
     // not staged), that block's q
     __shared__ uint32_t s_pwave[kEncWaves][3];
     __shared__ uint32_t s_abort;       // a bounded wait of this launch gave up
+    __shared__ __attribute__((aligned(16))) uint16_t s_cut[kKind == kEncCut ? kBlockElems : 1];
     __shared__ __attribute__((aligned(16))) uint32_t s_stage[kEncWaves][kEncStageWords];
 
     publish_seq(p.host_ctl, p.seq);
@@ -1810,11 +1884,14 @@ __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
             touch0 = *(const __attribute__((address_space(1))) uint32_t*)(k + 64u * (i0 < lines ? i0 : 0u));
             touch1 = *(const __attribute__((address_space(1))) uint32_t*)(k + 64u * (i1 < lines ? i1 : 0u));
         }
-        load_block_regs(p, cur, g, 2 * wave, lane, D0);
-        load_block_regs(p, cur, g, 2 * wave + 1, lane, D1);
+        load_block_from<kKind>(p, cur, g, 2 * wave, lane, D0, true);
+        load_block_from<kKind>(p, cur, g, 2 * wave + 1, lane, D1, true);
         uint32_t nan0, nan1;
-        keys0 = block_keys(D0, block_exists(g, cur.tile, 128 * wave + lane), nan0);
-        keys1 = block_keys(D1, block_exists(g, cur.tile, 128 * wave + 64 + lane), nan1);
+        keys0 = block_keys(D0, block_whole(g, cur.tile, 128 * wave + lane), nan0);
+        keys1 = block_keys(D1, block_whole(g, cur.tile, 128 * wave + 64 + lane), nan1);
+        if (kKind == kEncCut && has_cut_block(g, cur.tile, wave))
+            take_cut_block(g, job_of(p, cur).in, cur.tile, wave, lane, s_cut, D0, D1, keys0,
+                           keys1, nan0, nan1);
         if (fused)
             publish_keys2(p, cur.t, min(keys0 >> 16, keys1 >> 16),
                           max(keys0 & 0xFFFFu, keys1 & 0xFFFFu), s_min, s_max, wave, lane);
@@ -1861,10 +1938,8 @@ __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
             // unused), so that the loads are the same on every path.
             const TileCtx& lc = has_next ? nxt : cur;
             const Group& gl = p.groups[lc.gi];
-            load_block_from(p, lc, gl, wave_source(p, lc, gl, 2 * wave), 2 * wave, lane, Y0,
-                            has_next);
-            load_block_from(p, lc, gl, wave_source(p, lc, gl, 2 * wave + 1), 2 * wave + 1,
-                            lane, Y1, has_next);
+            load_block_from<kKind>(p, lc, gl, 2 * wave, lane, Y0, has_next);
+            load_block_from<kKind>(p, lc, gl, 2 * wave + 1, lane, Y1, has_next);
         }
 
         // c. the next tile's keys, while the reads above are in flight; each
@@ -1875,8 +1950,11 @@ __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
         uint32_t nkeys0 = 0, nkeys1 = 0, nnan0 = 0, nnan1 = 0;
         if (has_next) {
             const Group& gn = p.groups[nxt.gi];
-            nkeys0 = block_keys(Y0, block_exists(gn, nxt.tile, (int)blk0), nnan0);
-            nkeys1 = block_keys(Y1, block_exists(gn, nxt.tile, (int)blk0 + 64), nnan1);
+            nkeys0 = block_keys(Y0, block_whole(gn, nxt.tile, (int)blk0), nnan0);
+            nkeys1 = block_keys(Y1, block_whole(gn, nxt.tile, (int)blk0 + 64), nnan1);
+            if (kKind == kEncCut && has_cut_block(gn, nxt.tile, wave))
+                take_cut_block(gn, job_of(p, nxt).in, nxt.tile, wave, lane, s_cut, Y0, Y1,
+                               nkeys0, nkeys1, nnan0, nnan1);
             if (fused) {
                 const uint32_t kmin = wave_min(min(nkeys0 >> 16, nkeys1 >> 16));
                 const uint32_t kmax = wave_max(max(nkeys0 & 0xFFFFu, nkeys1 & 0xFFFFu));
@@ -2056,9 +2134,14 @@ __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
         // Only the first wave to mark a job writes host memory: the marks of
         // every wave of a saturated page would be a stream of small writes
         // across the link, most of them to one word.
-        const bool overflow = (wave_bytes >> 2) + 16u > (uint32_t)kEncStageWords;
+        // A block cut short quantizes its zeros wrongly when recip is not
+        // finite (0 * recip is NaN): its wave then goes the marked way as
+        // well, whatever its size.  Nor does it hold its value throughout.
+        const bool cut = kKind == kEncCut && has_cut_block(g, cur.tile, wave);
+        const bool overflow = (wave_bytes >> 2) + 16u > (uint32_t)kEncStageWords ||
+                              (cut && !(fabsf(recip) <= FLT_MAX));
         bool uniform = false;
-        if (overflow) {
+        if (overflow && !cut) {
             const uint32_t ukey = __builtin_amdgcn_readfirstlane(keys0);
             uniform = (ukey >> 16) == (ukey & 0xFFFFu) &&
                       __ballot(keys0 != ukey || keys1 != ukey) == 0ull;
@@ -2172,7 +2255,7 @@ __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
 template <int kQuant, bool kEarly>
 __global__ __launch_bounds__(kEncThreads)
 __attribute__((amdgpu_waves_per_eu(3, 3))) void compress_persistent_kernel(CompressParams p) {
-    compress_persistent<kQuant, kEarly>(p);
+    compress_persistent<kQuant, kEarly, kEncPlain>(p);
 }
 
 // The same with the job records in the kernel arguments (jobs_inline == 2).
@@ -2180,7 +2263,35 @@ template <int kQuant, bool kEarly>
 __global__ __launch_bounds__(kEncThreads)
 __attribute__((amdgpu_waves_per_eu(3, 3))) void compress_persistent_argtable_kernel(
     CompressParams p, ArgTable) {
-    compress_persistent<kQuant, kEarly>(p);
+    compress_persistent<kQuant, kEarly, kEncPlain>(p);
+}
+
+// The same for segments that end inside a block.
+template <int kQuant, bool kEarly>
+__global__ __launch_bounds__(kEncThreads)
+__attribute__((amdgpu_waves_per_eu(3, 3))) void compress_cut_kernel(CompressParams p) {
+    compress_persistent<kQuant, kEarly, kEncCut>(p);
+}
+
+template <int kQuant, bool kEarly>
+__global__ __launch_bounds__(kEncThreads)
+__attribute__((amdgpu_waves_per_eu(3, 3))) void compress_cut_argtable_kernel(
+    CompressParams p, ArgTable) {
+    compress_persistent<kQuant, kEarly, kEncCut>(p);
+}
+
+// The same for layers that a wave's run crosses.
+template <int kQuant, bool kEarly>
+__global__ __launch_bounds__(kEncThreads)
+__attribute__((amdgpu_waves_per_eu(3, 3))) void compress_split_kernel(CompressParams p) {
+    compress_persistent<kQuant, kEarly, kEncSplit>(p);
+}
+
+template <int kQuant, bool kEarly>
+__global__ __launch_bounds__(kEncThreads)
+__attribute__((amdgpu_waves_per_eu(3, 3))) void compress_split_argtable_kernel(
+    CompressParams p, ArgTable) {
+    compress_persistent<kQuant, kEarly, kEncSplit>(p);
 }
 
 // ---- relative-bound pre-pass (jobs too long for the fused exchange) -------
@@ -3295,33 +3406,39 @@ hipError_t launch_compress_pipelined(const CompressParams& p, uint32_t grid,
     if (!tile_plan_ok(p.groups, p.num_groups, p.total_tiles, grid, true,
                       readable_jobs(p, arg ? table_bytes : 0)))
         return hipErrorInvalidValue;
+    // The instantiation: look-back placement by the longest job, the kind by
+    // the segments (a segment with a layer map and whole layers of blocks has
+    // no cut block, so a launch is of one kind).
     uint32_t longest = 0;
-    for (int i = 0; i < p.num_groups; ++i) longest = std::max(longest, p.groups[i].tiles_per_job);
+    int kind = kEncPlain;
+    for (int i = 0; i < p.num_groups; ++i) {
+        const Group& g = p.groups[i];
+        longest = std::max(longest, g.tiles_per_job);
+        if (g.layers == nullptr && g.n % kBlockElems != 0)
+            kind = kEncCut;
+        else if (g.layers != nullptr && g.elements_per_layer % (64u * kBlockElems) != 0)
+            kind = kEncSplit;
+    }
+    const int which = (longest <= kEarlyLookbackTiles ? 2 : 0) + (p.quantizer ? 1 : 0);
     if (arg) {
-        void (*k)(CompressParams, ArgTable) =
-            longest <= kEarlyLookbackTiles
-                ? (p.quantizer ? compress_persistent_argtable_kernel<1, true>
-                               : compress_persistent_argtable_kernel<0, true>)
-                : (p.quantizer ? compress_persistent_argtable_kernel<1, false>
-                               : compress_persistent_argtable_kernel<0, false>);
-        return launch_argtable(k, grid, kEncThreads, stream, start, stop, p, table,
-                               table_bytes);
+        static void (*const kernels[3][4])(CompressParams, ArgTable) = {
+        {compress_persistent_argtable_kernel<0, false>, compress_persistent_argtable_kernel<1, false>,
+         compress_persistent_argtable_kernel<0, true>, compress_persistent_argtable_kernel<1, true>},
+        {compress_cut_argtable_kernel<0, false>, compress_cut_argtable_kernel<1, false>,
+         compress_cut_argtable_kernel<0, true>, compress_cut_argtable_kernel<1, true>},
+        {compress_split_argtable_kernel<0, false>, compress_split_argtable_kernel<1, false>,
+         compress_split_argtable_kernel<0, true>, compress_split_argtable_kernel<1, true>}};
+        return launch_argtable(kernels[kind][which], grid, kEncThreads, stream, start, stop, p,
+                               table, table_bytes);
     }
-    if (longest <= kEarlyLookbackTiles) {
-        if (p.quantizer)
-            launch_block(compress_persistent_kernel<1, true>, grid, kEncThreads, stream, start,
-                         stop, p);
-        else
-            launch_block(compress_persistent_kernel<0, true>, grid, kEncThreads, stream, start,
-                         stop, p);
-    } else {
-        if (p.quantizer)
-            launch_block(compress_persistent_kernel<1, false>, grid, kEncThreads, stream, start,
-                         stop, p);
-        else
-            launch_block(compress_persistent_kernel<0, false>, grid, kEncThreads, stream, start,
-                         stop, p);
-    }
+    static void (*const kernels[3][4])(CompressParams) = {
+        {compress_persistent_kernel<0, false>, compress_persistent_kernel<1, false>,
+         compress_persistent_kernel<0, true>, compress_persistent_kernel<1, true>},
+        {compress_cut_kernel<0, false>, compress_cut_kernel<1, false>,
+         compress_cut_kernel<0, true>, compress_cut_kernel<1, true>},
+        {compress_split_kernel<0, false>, compress_split_kernel<1, false>,
+         compress_split_kernel<0, true>, compress_split_kernel<1, true>}};
+    launch_block(kernels[kind][which], grid, kEncThreads, stream, start, stop, p);
     return hipGetLastError();
 }
 

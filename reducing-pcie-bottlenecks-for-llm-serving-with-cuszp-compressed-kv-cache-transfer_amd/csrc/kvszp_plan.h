@@ -138,6 +138,16 @@ KVSZP_PLAN_FN uint32_t weighted_run_start(const Group* groups, int num_groups,
     return first + (i < (double)tiles ? (uint32_t)i : tiles);
 }
 
+// The launches that the persistent encoder takes: blocks inside one layer,
+// jobs whose tiles number at most half its grid (its waits are then
+// cycle-free with margin while all its workgroups are resident), and no
+// negative bound (its short cut to a block's rate compares max|x| / (2 eb)
+// with a limit).
+inline bool persistent_encoder_takes(uint32_t grid, bool one_layer_blocks,
+                                     uint32_t max_tiles_per_job, bool negative_bound) {
+    return grid != 0 && one_layer_blocks && max_tiles_per_job <= grid / 2 && !negative_bound;
+}
+
 // ---- the relative-bound pre-pass ---------------------------------------------
 
 // Its workgroups take 1 to kMinMaxTilesPerWg consecutive tiles each, as many
@@ -221,7 +231,7 @@ struct Chunk {
     size_t g0, g1;
     uint64_t tiles;
     uint32_t max_tiles_per_job;
-    bool whole_blocks;  // every block whole and inside one layer
+    bool one_layer_blocks;  // every block inside one layer
 };
 
 // Splits `specs` into launches of at most kMaxGroups groups (the group
@@ -236,8 +246,7 @@ inline std::vector<Chunk> split_chunks(const std::vector<GroupSpec>& specs) {
             const uint32_t tpj = tiles_per_job_of(s.n);
             ch.tiles += (uint64_t)tpj * s.jobs;
             ch.max_tiles_per_job = std::max(ch.max_tiles_per_job, tpj);
-            if ((s.n % kBlockElems) != 0 || (s.layers && (s.epl % kBlockElems) != 0))
-                ch.whole_blocks = false;
+            if (s.layers && (s.epl % kBlockElems) != 0) ch.one_layer_blocks = false;
         }
         chunks.push_back(ch);
     }
