@@ -528,11 +528,12 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         if (relative)
             bound_mode = (!safe && !f32 && ch.max_tiles_per_job <= c->fused_tile_limit)
                              ? kBoundFused : kBoundPrepass;
+        const bool prepass = bound_mode == kBoundPrepass;
         const bool persistent =
-            !safe && !f32 && bound_mode != kBoundPrepass &&
-            persistent_encoder_takes(c->pipelined_grid, ch.one_layer_blocks,
-                                     ch.max_tiles_per_job, negative_bound);
-        const bool use_arg = persistent && arg_table;
+            !safe && !f32 &&
+            persistent_encoder_takes(c->pipelined_grid, ch, prepass, negative_bound);
+        const bool use_arg = persistent && arg_table &&
+                             !long_jobs(ch.plain_blocks, ch.max_tiles_per_job);
         if (!use_arg) {
             const int r = need_table();
             if (r) return r;
@@ -604,7 +605,8 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
             p.ticket = nullptr;
             const uint32_t grid = (uint32_t)std::min<uint64_t>(ch.tiles, c->pipelined_grid);
             p.slot_cus = persistent_slot_cus(ch.tiles, grid, c->cus, c->slot_mix);
-            e = launch_compress_pipelined(p, grid, stream, timing_start(c, rec),
+            e = launch_compress_pipelined(p, grid, stream,
+                                          prepass ? nullptr : timing_start(c, rec),
                                           timing_stop(c, rec), use_arg ? jobs.data() : nullptr,
                                           use_arg ? table_bytes : 0);
         } else {
@@ -1196,9 +1198,10 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
     p.bound_mode = bound_mode;
     p.quantizer = c->quantizer;
     p.aligned16 = aligned16 ? 1 : 0;
+    const Chunk chunk{0, 1, p.total_tiles, tiles_per_job, true, n % kBlockElems == 0};
     const bool persistent =
-        !schedule_safe && bound_mode != kBoundPrepass &&
-        persistent_encoder_takes(c->pipelined_grid, true, tiles_per_job, negative_bound);
+        !schedule_safe && persistent_encoder_takes(c->pipelined_grid, chunk,
+                                                   bound_mode == kBoundPrepass, negative_bound);
     if (persistent || bound_mode == kBoundFused) {
         p.abort_word = words + kScratchAbort / 8;
         p.wait_ticks = c->wait_ticks;

@@ -827,17 +827,27 @@ __device__ __forceinline__ void build_rows_hi(const uint32_t* d, uint32_t count,
 
 // A job's pre-pass result (minmax_kernel): the largest max key and inverted
 // min key over its shards, on every lane.  False when no shard was written.
-__device__ __forceinline__ bool prepass_words(const CompressParams& p, uint32_t job,
-                                              uint32_t& wmax, uint32_t& wmin) {
+// prepass_pair: this lane's shard.
+__device__ __forceinline__ const unsigned long long* prepass_pair(const CompressParams& p,
+                                                                  uint32_t job) {
     const uint32_t lane = __lane_id();
-    const unsigned long long* w =
-        p.job_minmax + (size_t)job * minmax_stride(p.minmax_shards) +
-        (lane < p.minmax_shards ? lane : 0u) * kMinMaxShardWords;
-    const unsigned long long a = w[0], b = w[1];
+    return p.job_minmax + (size_t)job * minmax_stride(p.minmax_shards) +
+           (lane < p.minmax_shards ? lane : 0u) * kMinMaxShardWords;
+}
+
+__device__ __forceinline__ bool reduce_prepass(const CompressParams& p, unsigned long long a,
+                                               unsigned long long b, uint32_t& wmax,
+                                               uint32_t& wmin) {
     const bool written = (uint32_t)(a >> 32) == p.epoch && (uint32_t)(b >> 32) == p.epoch;
     wmax = wave_max(written ? (uint32_t)a : 0u);
     wmin = wave_max(written ? (uint32_t)b : 0u);
     return __ballot(written) != 0ull;
+}
+
+__device__ __forceinline__ bool prepass_words(const CompressParams& p, uint32_t job,
+                                              uint32_t& wmax, uint32_t& wmin) {
+    const unsigned long long* w = prepass_pair(p, job);
+    return reduce_prepass(p, w[0], w[1], wmax, wmin);
 }
 
 // kIn = 0: BF16 pages (any bound mode, layer maps); kIn = 1: contiguous
@@ -1309,6 +1319,11 @@ enum : int {
     // A segment ends inside a block (then there is no layer map).  256 segments
     // of 100003 values: 28.5 us, one workgroup per tile 41 us.
     kEncCut = 1,
+    // Jobs of more than 256 tiles, which the exchange does not take
+    // (long_jobs).  Two segments of 32 Mi values, pre-pass included: 98 us, one
+    // workgroup per tile 137 us; of 2.1 Mi values (260 tiles each) 16.9 us, 17.8.
+    // Look-back windows of 256 or 512 tiles instead of 64 took 104 and 111 us.
+    kEncLong = 3,
     // Layers that are no whole number of runs.  128 blocks of 36 layers of
     // 6400 values: 57.5 us, with each lane mapping its own block 59.3 us.
     kEncSplit = 2,
@@ -1925,14 +1940,21 @@ __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
         // read), so the wait for the read counts only the read.
         const unsigned long long* paddr = &p.tile_state[cur.t];
         if (wave == 0) {
-            if (fused)
-                paddr = &p.tile_minmax[cur.t - cur.tile +
-                                       min((uint32_t)lane, g.tiles_per_job - 1u)];
+            if (kKind == kEncLong ? p.bound_mode == kBoundPrepass : fused)
+                paddr = kKind == kEncLong
+                            ? prepass_pair(p, cur.job)
+                            : &p.tile_minmax[cur.t - cur.tile +
+                                             min((uint32_t)lane, g.tiles_per_job - 1u)];
         } else if (pending) {
             const PendingTile& q = s_pend[parity ^ 1u];
             paddr = lookback_first_addr(p.tile_state, q.t, q.tile);
         }
         const unsigned long long probe = load_relaxed(paddr);
+        // kEncLong: the second word of wave 0's pair (the same word again
+        // otherwise, so that the loads are the same on every path)
+        unsigned long long probe2 = 0;
+        if constexpr (kKind == kEncLong)
+            probe2 = load_relaxed(paddr + (wave == 0 && p.bound_mode == kBoundPrepass ? 1 : 0));
         {
             // Without a next tile the loads read the zero block (values
             // unused), so that the loads are the same on every path.
@@ -1971,11 +1993,18 @@ __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
             const float eps = job_of(p, cur).eps;
             float eb = eps;
             uint32_t fast = 0;
-            if (fused) {
+            if (kKind == kEncLong ? p.bound_mode == kBoundPrepass : fused) {
                 uint32_t kmin, kmax;
-                if (job_keys(p, cur.t - cur.tile, g.tiles_per_job, lane, kmin, kmax, true, probe,
-                             bound) && lane == 0)
+                if constexpr (kKind == kEncLong) {
+                    uint32_t wmax, wmin;
+                    if (!reduce_prepass(p, probe, probe2, wmax, wmin) && lane == 0)
+                        flag_error(p.error, p.error_marker, kErrSpin);
+                    kmax = wmax;
+                    kmin = 0xFFFFu - wmin;
+                } else if (job_keys(p, cur.t - cur.tile, g.tiles_per_job, lane, kmin, kmax, true,
+                                    probe, bound) && lane == 0) {
                     s_abort = 1;
+                }
                 eb = relative_bound(eps, kmin, kmax);
                 const float jabs = fmaxf(fabsf(min_key_value(kmin)), fabsf(max_key_value(kmax)));
                 fast = jabs * (0.5f / eb) <= kFastLimit ? 1u : 0u;
@@ -2278,6 +2307,13 @@ __global__ __launch_bounds__(kEncThreads)
 __attribute__((amdgpu_waves_per_eu(3, 3))) void compress_cut_argtable_kernel(
     CompressParams p, ArgTable) {
     compress_persistent<kQuant, kEarly, kEncCut>(p);
+}
+
+// The same for long jobs.
+template <int kQuant>
+__global__ __launch_bounds__(kEncThreads)
+__attribute__((amdgpu_waves_per_eu(3, 3))) void compress_long_kernel(CompressParams p) {
+    compress_persistent<kQuant, false, kEncLong>(p);
 }
 
 // The same for layers that a wave's run crosses.
@@ -3411,14 +3447,23 @@ hipError_t launch_compress_pipelined(const CompressParams& p, uint32_t grid,
     // no cut block, so a launch is of one kind).
     uint32_t longest = 0;
     int kind = kEncPlain;
+    bool plain = true;
     for (int i = 0; i < p.num_groups; ++i) {
         const Group& g = p.groups[i];
         longest = std::max(longest, g.tiles_per_job);
+        plain = plain && g.layers == nullptr && g.n % kBlockElems == 0;
         if (g.layers == nullptr && g.n % kBlockElems != 0)
             kind = kEncCut;
         else if (g.layers != nullptr && g.elements_per_layer % (64u * kBlockElems) != 0)
             kind = kEncSplit;
     }
+    if (long_jobs(plain, longest)) {
+        if (arg) return hipErrorInvalidValue;
+        launch_block(p.quantizer ? compress_long_kernel<1> : compress_long_kernel<0>, grid,
+                     kEncThreads, stream, start, stop, p);
+        return hipGetLastError();
+    }
+    if (p.bound_mode == kBoundPrepass) return hipErrorInvalidValue;
     const int which = (longest <= kEarlyLookbackTiles ? 2 : 0) + (p.quantizer ? 1 : 0);
     if (arg) {
         static void (*const kernels[3][4])(CompressParams, ArgTable) = {

@@ -138,16 +138,6 @@ KVSZP_PLAN_FN uint32_t weighted_run_start(const Group* groups, int num_groups,
     return first + (i < (double)tiles ? (uint32_t)i : tiles);
 }
 
-// The launches that the persistent encoder takes: blocks inside one layer,
-// jobs whose tiles number at most half its grid (its waits are then
-// cycle-free with margin while all its workgroups are resident), and no
-// negative bound (its short cut to a block's rate compares max|x| / (2 eb)
-// with a limit).
-inline bool persistent_encoder_takes(uint32_t grid, bool one_layer_blocks,
-                                     uint32_t max_tiles_per_job, bool negative_bound) {
-    return grid != 0 && one_layer_blocks && max_tiles_per_job <= grid / 2 && !negative_bound;
-}
-
 // ---- the relative-bound pre-pass ---------------------------------------------
 
 // Its workgroups take 1 to kMinMaxTilesPerWg consecutive tiles each, as many
@@ -232,7 +222,28 @@ struct Chunk {
     uint64_t tiles;
     uint32_t max_tiles_per_job;
     bool one_layer_blocks;  // every block inside one layer
+    bool plain_blocks;      // every block whole, no layer map
 };
+
+// Launches whose jobs are too long for the exchange (more than kTileBlocks
+// tiles): the persistent encoder for long jobs, built for whole blocks without
+// a layer map, takes the bound from the pre-pass or as given, and a tile waits
+// for earlier tiles only.
+inline bool long_jobs(bool plain_blocks, uint32_t max_tiles_per_job) {
+    return plain_blocks && max_tiles_per_job > (uint32_t)kTileBlocks;
+}
+
+// The launches that the persistent encoder takes: long jobs as above, and jobs
+// of blocks inside one layer whose tiles number at most half its grid (its
+// waits are then cycle-free with margin while all its workgroups are
+// resident), unless the bound comes from the pre-pass.  None with a negative
+// bound: its short cut to a block's rate compares max|x| / (2 eb) with a limit.
+inline bool persistent_encoder_takes(uint32_t grid, const Chunk& ch, bool prepass,
+                                     bool negative_bound) {
+    if (grid == 0 || negative_bound) return false;
+    if (long_jobs(ch.plain_blocks, ch.max_tiles_per_job)) return true;
+    return !prepass && ch.one_layer_blocks && ch.max_tiles_per_job <= grid / 2;
+}
 
 // Splits `specs` into launches of at most kMaxGroups groups (the group
 // records travel as kernel arguments).  The reference takes any number of
@@ -240,13 +251,14 @@ struct Chunk {
 inline std::vector<Chunk> split_chunks(const std::vector<GroupSpec>& specs) {
     std::vector<Chunk> chunks;
     for (size_t g0 = 0; g0 < specs.size(); g0 += kMaxGroups) {
-        Chunk ch{g0, std::min(specs.size(), g0 + (size_t)kMaxGroups), 0, 0, true};
+        Chunk ch{g0, std::min(specs.size(), g0 + (size_t)kMaxGroups), 0, 0, true, true};
         for (size_t gi = ch.g0; gi < ch.g1; ++gi) {
             const GroupSpec& s = specs[gi];
             const uint32_t tpj = tiles_per_job_of(s.n);
             ch.tiles += (uint64_t)tpj * s.jobs;
             ch.max_tiles_per_job = std::max(ch.max_tiles_per_job, tpj);
             if (s.layers && (s.epl % kBlockElems) != 0) ch.one_layer_blocks = false;
+            if (s.layers || (s.n % kBlockElems) != 0) ch.plain_blocks = false;
         }
         chunks.push_back(ch);
     }
