@@ -479,7 +479,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
     const bool relative = c->config.use_relative_error != 0 && !bounds_given;
     // Workspaces.
     if ((rc = ensure(c->tile_state, max_tiles * 8, true, stream)) ||
-        (rc = ensure(c->tile_minmax, max_tiles * 8, true, stream)) ||
+        (rc = ensure(c->tile_minmax, max_tiles * (f32 ? 16 : 8), true, stream)) ||
         (rc = ensure(c->job_minmax, minmax_words * 8, true, stream)) ||
         (rc = ensure(c->job_flags, batch * 4, true, stream)) ||
         (rc = ensure_host_results(c, batch * 12)))
@@ -526,7 +526,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         p.minmax_shards = minmax_shards(ch.tiles, ch.max_tiles_per_job, batch, UINT64_MAX);
         int bound_mode = kBoundAbsolute;
         if (relative)
-            bound_mode = (!safe && !f32 && ch.max_tiles_per_job <= c->fused_tile_limit)
+            bound_mode = (!safe && ch.max_tiles_per_job <= c->fused_tile_limit)
                              ? kBoundFused : kBoundPrepass;
         const bool prepass = bound_mode == kBoundPrepass;
         const bool persistent =
@@ -621,7 +621,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
     // A recent give-up on this context: the schedule that needs no residency
     // for this call too (the device is likely still shared).
     bool schedule_safe = safe;
-    if (!safe && !f32 && c->safe_left > 0) {
+    if (!safe && c->safe_left > 0) {
         c->safe_left -= 1;
         c->safe_calls += 1;
         schedule_safe = true;

@@ -100,7 +100,7 @@ struct DecompressJob {
 struct CompressParams {
     const CompressJob* jobs;
     unsigned long long* tile_state;   // look-back words, one per tile
-    unsigned long long* tile_minmax;  // fused min/max words, one per tile
+    unsigned long long* tile_minmax;  // fused min/max words, one per tile (fp32: two)
     const unsigned long long* job_minmax;  // pre-pass words (minmax_stride per job)
     uint32_t minmax_shards;
     uint32_t* host_sizes;             // out (pinned host): stream bytes per job

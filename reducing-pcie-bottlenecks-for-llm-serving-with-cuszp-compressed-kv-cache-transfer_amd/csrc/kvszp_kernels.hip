@@ -359,6 +359,40 @@ __device__ __forceinline__ float relative_bound_f32(float eps, uint32_t kmin,
     return eps * range;
 }
 
+// Order keys of the 32 fp32 values in d[], as minmax_kernel<1> keeps them: the
+// smallest non-NaN key, and the largest key with kKey32Nan for a NaN.  Read
+// as signed numbers, the patterns with the sign bit clear order by value and
+// lie above all others; read as unsigned numbers, those with the sign bit set
+// lie above all others and order by magnitude (see block_keys): two maxima
+// over the raw words serve a set that holds both signs and no NaN.
+// Of the first `count` values only, when the block is cut short.
+__device__ __forceinline__ void keys32_minmax(const uint32_t* d, uint32_t count,
+                                              uint32_t& kmin, uint32_t& kmax) {
+    int32_t smax = INT32_MIN;
+    uint32_t umax = 0;
+#pragma unroll
+    for (int v = 0; v < kBlockElems; ++v) {
+        smax = max(smax, (int32_t)d[v]);
+        umax = max(umax, d[v]);
+    }
+    if (count == kBlockElems && smax >= 0 && smax <= 0x7F800000 && umax >= 0x80000000u && umax <= 0xFF800000u) {
+        kmin = ~umax;
+        kmax = (uint32_t)smax | 0x80000000u;
+        return;
+    }
+    kmin = 0xFFFFFFFFu;
+    kmax = 0u;
+#pragma unroll
+    for (int v = 0; v < kBlockElems; ++v) {
+        const float x = __uint_as_float(d[v]);
+        const uint32_t k = x != x ? kKey32Nan : key32(x);
+        if ((uint32_t)v < count) {
+            kmax = max(kmax, k);
+            if (x == x) kmin = min(kmin, k);
+        }
+    }
+}
+
 // ---- layer-index gather ----------------------------------------------------
 
 // selected_bf16_source_index (cu:33-50) for an arbitrary logical index.
@@ -523,6 +557,47 @@ __device__ __forceinline__ void load_block_f32(const float* in, uint64_t e0,
     const __attribute__((address_space(1))) uint32_t* g =
         (const __attribute__((address_space(1))) uint32_t*)(in + e0);
     for (uint32_t v = 0; v < count; ++v) d[v] = g[v];
+}
+
+// The 32 fp32 values of each lane's block, the wave's first block at element
+// E: whole waves read 1 KiB per instruction and exchange through their 1024
+// LDS words `stage`, 32 blocks at a time (the layout of store_wave_f32);
+// others block by block.
+__device__ __forceinline__ void load_wave_f32(const float* in, uint64_t E, uint64_t n,
+                                              uint32_t count, uint32_t* d, uint32_t* stage,
+                                              int lane) {
+    if (E + 64u * kBlockElems > n) {
+        load_block_f32(in, E + (uint32_t)lane * kBlockElems, count, d);
+        return;
+    }
+    const g_u32* src = to_global(reinterpret_cast<const uint32_t*>(in + E)) + 4 * lane;
+    u32x4 v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = *(const g_u32x4_a4*)(src + 256 * i);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t j = 64u * i + (uint32_t)lane, b = j >> 3, c = j & 7u;
+            *reinterpret_cast<u32x4*>(stage + 4u * (8u * b + (c ^ (b & 7u)))) = v[4 * r + i];
+        }
+        __builtin_amdgcn_wave_barrier();
+        __asm__ volatile("" ::: "memory");
+        if ((lane >> 5) == r) {
+            const uint32_t b = (uint32_t)lane & 31u;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const u32x4 q = *reinterpret_cast<const u32x4*>(
+                    stage + 4u * (8u * b + ((uint32_t)c ^ (b & 7u))));
+                d[4 * c + 0] = q.x;
+                d[4 * c + 1] = q.y;
+                d[4 * c + 2] = q.z;
+                d[4 * c + 3] = q.w;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        __asm__ volatile("" ::: "memory");  // before the words are reused
+    }
 }
 
 // ---- workgroup scan + decoupled look-back ---------------------------------
@@ -850,8 +925,142 @@ __device__ __forceinline__ bool prepass_words(const CompressParams& p, uint32_t 
     return reduce_prepass(p, w[0], w[1], wmax, wmin);
 }
 
-// kIn = 0: BF16 pages (any bound mode, layer maps); kIn = 1: contiguous
-// fp32 pages (absolute or pre-pass bound), the single-page fp32 API.
+// The fused bound exchange of the one-workgroup-per-tile kernels: each lane's
+// min/max keys in, the job's out (on every thread).  The tile's keys go out as
+// one epoch-tagged word (BF16) or two (fp32: max key, min key), and each
+// thread reads those of one tile of the job; the host guarantees that a job
+// has at most kThreads tiles and that they can be co-resident.  True when a
+// time-bounded wait gave up (on every thread).
+template <int kIn>
+__device__ __forceinline__ bool exchange_minmax(const CompressParams& p, const Group& g,
+                                                uint32_t t, uint32_t tile, uint32_t& kmin,
+                                                uint32_t& kmax, uint32_t* s_min,
+                                                uint32_t* s_max, uint32_t* s_abort,
+                                                const WaitBound& bound) {
+    constexpr uint32_t kEmptyMin = kIn ? 0xFFFFFFFFu : kKeyEmptyMin;
+    constexpr int kWords = kIn ? 2 : 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    kmin = wave_min(kmin);
+    kmax = wave_max(kmax);
+    if (lane == 0) {
+        s_min[wave] = kmin;
+        s_max[wave] = kmax;
+    }
+    __syncthreads();
+    if (tid < kWords) {
+#pragma unroll
+        for (int w = 0; w < kThreads / 64; ++w) {
+            kmin = min(kmin, s_min[w]);
+            kmax = max(kmax, s_max[w]);
+        }
+        const uint32_t word = kIn ? (tid == 0 ? kmax : kmin) : (kmin << 16) | kmax;
+        store_relaxed(&p.tile_minmax[(size_t)t * kWords + tid],
+                      ((unsigned long long)p.epoch << 32) | word);
+    }
+    kmin = kEmptyMin;
+    kmax = 0u;
+    if ((uint32_t)tid < g.tiles_per_job) {
+        const unsigned long long* slot = &p.tile_minmax[(size_t)(t - tile + tid) * kWords];
+        unsigned long long w = load_relaxed(slot), w2 = load_relaxed(slot + (kWords - 1));
+        uint64_t deadline = 0;
+        for (uint32_t spins = 0;
+             (uint32_t)(w >> 32) != p.epoch || (uint32_t)(w2 >> 32) != p.epoch; ++spins) {
+            if (bound.word != nullptr) {
+                if (wait_gives_up(bound, deadline, spins)) {
+                    *s_abort = 1;
+                    break;
+                }
+            } else if (spins >= kSpinLimit) {
+                flag_error(p.error, p.error_marker, kErrSpin);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+            w = load_relaxed(slot);
+            w2 = load_relaxed(slot + (kWords - 1));
+        }
+        kmin = kIn ? (uint32_t)w2 : (uint32_t)(w >> 16) & 0xFFFFu;
+        kmax = kIn ? (uint32_t)w : (uint32_t)w & 0xFFFFu;
+    }
+    kmin = wave_min(kmin);
+    kmax = wave_max(kmax);
+    __syncthreads();  // s_min/s_max reuse
+    if (*s_abort) return true;  // the launch gave up; the host encodes again
+    if (lane == 0) {
+        s_min[wave] = kmin;
+        s_max[wave] = kmax;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) {
+        kmin = min(kmin, s_min[w]);
+        kmax = max(kmax, s_max[w]);
+    }
+    return false;
+}
+
+// A wave's payload staged in LDS: the block is words [off, off + count) of
+// the wave's payload.  The stream words are the transposed rows P:
+// w_j = P[j] (kSignHi false), or w_0 = P[15] and w_j = P[j - 1] (sign-high
+// rows).  Words are written from the highest index down: a lane's unused
+// slots (index >= count) only ever fall on words of later blocks, which are
+// written afterwards, or past the payload end, so `stage` needs room for
+// the payload plus 16 words.
+template <bool kSignHi>
+__device__ __forceinline__ void stage_payload(const uint32_t* P, uint32_t count,
+                                              uint32_t off, uint32_t cmax,
+                                              uint32_t* stage) {
+    __asm__ volatile("" ::: "memory");
+    if (count) {
+        uint32_t* s = stage + off;
+#pragma unroll
+        for (int j = 15; j >= 0; --j)
+            if ((uint32_t)j < cmax) s[j] = kSignHi ? P[(j + 15) & 15] : P[j];
+    }
+    __asm__ volatile("" ::: "memory");
+}
+
+// Writes a wave's staged payload (`words` words) to `dst` (4-byte aligned):
+// lane l moves words 4l .. 4l + 3 of every 256-word chunk with one 16-byte
+// LDS read and one 16-byte store (each store instruction covers 1 KiB of
+// contiguous stream), then lanes 0..2 the last words.
+__device__ __forceinline__ void copy_payload(uint32_t* dst, uint32_t words,
+                                             const uint32_t* stage, int lane) {
+    __builtin_amdgcn_wave_barrier();
+    __asm__ volatile("" ::: "memory");
+    g_u32* d = to_global(dst);
+    const uint32_t quads = words >> 2;
+    for (uint32_t q = (uint32_t)lane; q < quads; q += 64u)
+        *(g_u32x4_a4*)(d + 4u * q) = *(const u32x4*)(stage + 4u * q);
+    const uint32_t tail = 4u * quads + (uint32_t)lane;
+    if (tail < words) d[tail] = stage[tail];
+    __builtin_amdgcn_wave_barrier();
+    __asm__ volatile("" ::: "memory");  // before the words are reused
+}
+
+// A wave's payload from its transposed rows, for rates of at most 15 and at
+// most kWaveStage words: through LDS, 1 KiB per store instruction.  `dst` is
+// the tile's payload, `excl` and `bytes` this lane's place in it, `outlier`
+// the word in front of the block's words (when has_o).  False, and nothing
+// written, when the wave does not qualify.
+constexpr uint32_t kWaveStage = 1024;
+
+__device__ __forceinline__ bool store_wave_payload(uint32_t* dst, uint32_t excl, uint32_t bytes,
+                                                   uint32_t count, uint32_t rmax, bool has_o,
+                                                   uint32_t outlier, const uint32_t* P,
+                                                   uint32_t* stage, int lane) {
+    const uint32_t first = __builtin_amdgcn_readfirstlane(excl);
+    const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)(excl + bytes), 63);
+    const uint32_t words = (end - first) >> 2;
+    if (rmax > 15u || words > kWaveStage) return false;
+    const uint32_t off = (excl - first) >> 2;
+    stage_payload<false>(P, count, off + (has_o ? 1u : 0u), rmax + 1u, stage);
+    if (has_o) stage[off] = outlier;  // after the lanes whose unused slots fall there
+    copy_payload(dst + (first >> 2), words, stage, lane);
+    return true;
+}
+
+// kIn = 0: BF16 pages (layer maps too); kIn = 1: contiguous fp32 pages, the
+// single-page fp32 API.
 template <int kQuant, int kIn>
 __global__ __launch_bounds__(kThreads) void compress_kernel(CompressParams p) {
     __shared__ uint32_t s_tile;
@@ -861,7 +1070,8 @@ __global__ __launch_bounds__(kThreads) void compress_kernel(CompressParams p) {
     __shared__ uint32_t s_prefix;
     __shared__ uint32_t s_abort;
     __shared__ uint8_t s_rate[kTileBlocks];
-    __shared__ __attribute__((aligned(16))) uint32_t s_stage[kThreads / 64][1024];  // 4 KiB per wave
+    // load exchange, payload staging (stage_payload needs 16 words of slack)
+    __shared__ __attribute__((aligned(16))) uint32_t s_stage[kThreads / 64][kWaveStage + 16];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -892,84 +1102,30 @@ __global__ __launch_bounds__(kThreads) void compress_kernel(CompressParams p) {
     uint32_t bad = 0;
     uint32_t d[kIn ? kBlockElems : kBlockElems / 2];
     if constexpr (kIn)
-        load_block_f32(reinterpret_cast<const float*>(J.in), e0, count, d);
+        load_wave_f32(reinterpret_cast<const float*>(J.in),
+                      tile_first + (uint32_t)wave * 64u * kBlockElems, n, count, d,
+                      &s_stage[wave][0], lane);
     else
         load_block_wave(g, J.in, tile_first, (uint32_t)tid * kBlockElems, count,
                         p.aligned16 != 0, d, &bad, &s_stage[wave][0]);
 
     float eb = J.eps;
-    if constexpr (kIn) {
-        if (p.bound_mode != kBoundAbsolute) {  // pre-pass words (32-bit keys)
-            uint32_t wmax, wmin;
-            if (!prepass_words(p, job, wmax, wmin)) bad |= 2;
-            eb = relative_bound_f32(J.eps, 0xFFFFFFFFu - wmin, wmax);
-        }
-    } else if (p.bound_mode != kBoundAbsolute) {
+    if (p.bound_mode != kBoundAbsolute) {
         uint32_t kmin, kmax;
         if (p.bound_mode == kBoundFused) {
-            block_key_minmax(d, count, kmin, kmax);
-            kmin = wave_min(kmin);
-            kmax = wave_max(kmax);
-            if (lane == 0) {
-                s_min[wave] = kmin;
-                s_max[wave] = kmax;
-            }
-            __syncthreads();
-            if (tid == 0) {
-#pragma unroll
-                for (int w = 1; w < kThreads / 64; ++w) {
-                    kmin = s_min[w] < kmin ? s_min[w] : kmin;
-                    kmax = s_max[w] > kmax ? s_max[w] : kmax;
-                }
-                store_relaxed(&p.tile_minmax[t],
-                              ((unsigned long long)p.epoch << 32) |
-                                  (kmin << 16) | kmax);
-            }
-            // Exchange with every tile of this job (host guarantees
-            // tiles_per_job <= kThreads and that they can be co-resident).
-            kmin = kKeyEmptyMin;
-            kmax = kKeyEmptyMax;
-            if ((uint32_t)tid < g.tiles_per_job) {
-                const unsigned long long* slot = &p.tile_minmax[t - tile + tid];
-                unsigned long long w = load_relaxed(slot);
-                uint64_t deadline = 0;
-                for (uint32_t spins = 0; (uint32_t)(w >> 32) != p.epoch; ++spins) {
-                    if (bound.word != nullptr) {
-                        if (wait_gives_up(bound, deadline, spins)) {
-                            s_abort = 1;
-                            break;
-                        }
-                    } else if (spins >= kSpinLimit) {
-                        flag_error(p.error, p.error_marker, kErrSpin);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                    w = load_relaxed(slot);
-                }
-                kmin = (uint32_t)(w >> 16) & 0xFFFFu;
-                kmax = (uint32_t)w & 0xFFFFu;
-            }
-            kmin = wave_min(kmin);
-            kmax = wave_max(kmax);
-            __syncthreads();  // s_min/s_max reuse
-            if (s_abort) return;  // the launch gave up; the host encodes again
-            if (lane == 0) {
-                s_min[wave] = kmin;
-                s_max[wave] = kmax;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int w = 0; w < kThreads / 64; ++w) {
-                kmin = s_min[w] < kmin ? s_min[w] : kmin;
-                kmax = s_max[w] > kmax ? s_max[w] : kmax;
-            }
+            if constexpr (kIn)
+                keys32_minmax(d, count, kmin, kmax);
+            else
+                block_key_minmax(d, count, kmin, kmax);
+            if (exchange_minmax<kIn>(p, g, t, tile, kmin, kmax, s_min, s_max, &s_abort, bound))
+                return;
         } else {
             uint32_t wmax, wmin;
             if (!prepass_words(p, job, wmax, wmin)) bad |= 2;  // reported as a spin error below
             kmax = wmax;
-            kmin = 0xFFFFu - wmin;
+            kmin = (kIn ? 0xFFFFFFFFu : 0xFFFFu) - wmin;
         }
-        eb = relative_bound(J.eps, kmin, kmax);
+        eb = kIn ? relative_bound_f32(J.eps, kmin, kmax) : relative_bound(J.eps, kmin, kmax);
     }
     const float recip = 0.5f / eb;  // cu:166, IEEE division
 
@@ -1027,9 +1183,13 @@ __global__ __launch_bounds__(kThreads) void compress_kernel(CompressParams p) {
     // Payload (cu:302-358): sign word, then `rate` plane words.
     const uint32_t rmax = wave_max(rate);
     if (rmax == 0) return;
-    uint32_t* dst = reinterpret_cast<uint32_t*>(J.out + R + s_prefix + sc.exclusive);
     const uint32_t count_words = rate ? rate + 1u : 0u;
     transpose16x2(P);  // rows 0..15 = words w_0..w_15
+    if constexpr (kIn)
+        if (store_wave_payload(reinterpret_cast<uint32_t*>(J.out + R + s_prefix), sc.exclusive,
+                               bytes, count_words, rmax, false, 0u, P, &s_stage[wave][0], lane))
+            return;
+    uint32_t* dst = reinterpret_cast<uint32_t*>(J.out + R + s_prefix + sc.exclusive);
     store_words<16>(dst, P, count_words < 16u ? count_words : 16u,
                     rmax < 15u ? rmax + 1u : 16u);
     if (rmax >= 16u) {
@@ -1126,14 +1286,17 @@ __device__ __forceinline__ uint32_t residual_plane31(const uint32_t* c) {
     return w;
 }
 
-// One workgroup per tile, one block per thread, contiguous fp32 pages with
-// an absolute or pre-pass bound (the schedule of compress_kernel).
+// One workgroup per tile, one block per thread, contiguous fp32 pages (the
+// schedule of compress_kernel).
 template <int kQuant, int kMode>
 __global__ __launch_bounds__(kThreads) void compress_lorenzo_kernel(CompressParams p) {
     __shared__ uint32_t s_tile;
     __shared__ uint32_t s_wave[kThreads / 64];
     __shared__ uint32_t s_prefix;
     __shared__ uint32_t s_abort;
+    __shared__ uint32_t s_min[kThreads / 64];
+    __shared__ uint32_t s_max[kThreads / 64];
+    __shared__ __attribute__((aligned(16))) uint32_t s_stage[kThreads / 64][kWaveStage + 16];
     __shared__ uint8_t s_hdr[kTileBlocks];
 
     const int tid = threadIdx.x;
@@ -1161,13 +1324,24 @@ __global__ __launch_bounds__(kThreads) void compress_lorenzo_kernel(CompressPara
         b < nb ? (uint32_t)(n - e0 < kBlockElems ? n - e0 : kBlockElems) : 0u;
 
     uint32_t d[kBlockElems];
-    load_block_f32(reinterpret_cast<const float*>(J.in), e0, count, d);
+    load_wave_f32(reinterpret_cast<const float*>(J.in),
+                  (uint64_t)tile * kTileElems + (uint32_t)wave * 64u * kBlockElems, n, count, d,
+                  s_stage[wave], lane);
     float eb = J.eps;
     uint32_t bad = 0;
-    if (p.bound_mode != kBoundAbsolute) {  // pre-pass words (32-bit keys)
-        uint32_t wmax, wmin;
-        if (!prepass_words(p, job, wmax, wmin)) bad = 1;
-        eb = relative_bound_f32(J.eps, 0xFFFFFFFFu - wmin, wmax);
+    if (p.bound_mode != kBoundAbsolute) {
+        uint32_t kmin, kmax;
+        if (p.bound_mode == kBoundFused) {
+            keys32_minmax(d, count, kmin, kmax);
+            if (exchange_minmax<1>(p, g, t, tile, kmin, kmax, s_min, s_max, &s_abort, bound))
+                return;
+        } else {
+            uint32_t wmax, wmin;
+            if (!prepass_words(p, job, wmax, wmin)) bad = 1;
+            kmax = wmax;
+            kmin = 0xFFFFFFFFu - wmin;
+        }
+        eb = relative_bound_f32(J.eps, kmin, kmax);
     }
     const float recip = 0.5f / eb;  // IEEE division, as in fixed mode
 
@@ -1212,15 +1386,17 @@ __global__ __launch_bounds__(kThreads) void compress_lorenzo_kernel(CompressPara
     __syncthreads();
     if (s_abort) return;
 
-    uint32_t* dst = reinterpret_cast<uint32_t*>(J.out + R + s_prefix + sc.exclusive);
-    if (has_o) *to_global(dst) = outlier;
-    dst += has_o ? 1 : 0;
     const uint32_t rmax = wave_max(rate);
-    if (rmax == 0) return;
     const uint32_t count_words = rate ? rate + 1u : 0u;
     uint32_t P[16];
     residual_rows_lo(d, P);
     transpose16x2(P);  // rows 0..15 = words w_0..w_15
+    if (store_wave_payload(reinterpret_cast<uint32_t*>(J.out + R + s_prefix), sc.exclusive, bytes,
+                           count_words, rmax, has_o, outlier, P, s_stage[wave], lane))
+        return;
+    uint32_t* dst = reinterpret_cast<uint32_t*>(J.out + R + s_prefix + sc.exclusive);
+    if (has_o) *to_global(dst) = outlier;
+    dst += has_o ? 1 : 0;
     store_words<16>(dst, P, count_words < 16u ? count_words : 16u,
                     rmax < 15u ? rmax + 1u : 16u);
     if (rmax >= 16u) {
@@ -1713,45 +1889,6 @@ __device__ __forceinline__ void publish_keys2(const CompressParams& p, uint32_t 
         store_relaxed(&p.tile_minmax[t],
                       ((unsigned long long)p.epoch << 32) | (kmin << 16) | kmax);
     }
-}
-
-// A wave's payload staged in LDS: the block is words [off, off + count) of
-// the wave's payload.  The stream words are the transposed rows P:
-// w_j = P[j] (kSignHi false), or w_0 = P[15] and w_j = P[j - 1] (sign-high
-// rows).  Words are written from the highest index down: a lane's unused
-// slots (index >= count) only ever fall on words of later blocks, which are
-// written afterwards, or past the payload end, so `stage` needs room for
-// the payload plus 16 words.
-template <bool kSignHi>
-__device__ __forceinline__ void stage_payload(const uint32_t* P, uint32_t count,
-                                              uint32_t off, uint32_t cmax,
-                                              uint32_t* stage) {
-    __asm__ volatile("" ::: "memory");
-    if (count) {
-        uint32_t* s = stage + off;
-#pragma unroll
-        for (int j = 15; j >= 0; --j)
-            if ((uint32_t)j < cmax) s[j] = kSignHi ? P[(j + 15) & 15] : P[j];
-    }
-    __asm__ volatile("" ::: "memory");
-}
-
-// Writes a wave's staged payload (`words` words) to `dst` (4-byte aligned):
-// lane l moves words 4l .. 4l + 3 of every 256-word chunk with one 16-byte
-// LDS read and one 16-byte store (each store instruction covers 1 KiB of
-// contiguous stream), then lanes 0..2 the last words.
-__device__ __forceinline__ void copy_payload(uint32_t* dst, uint32_t words,
-                                             const uint32_t* stage, int lane) {
-    __builtin_amdgcn_wave_barrier();
-    __asm__ volatile("" ::: "memory");
-    g_u32* d = to_global(dst);
-    const uint32_t quads = words >> 2;
-    for (uint32_t q = (uint32_t)lane; q < quads; q += 64u)
-        *(g_u32x4_a4*)(d + 4u * q) = *(const u32x4*)(stage + 4u * q);
-    const uint32_t tail = 4u * quads + (uint32_t)lane;
-    if (tail < words) d[tail] = stage[tail];
-    __builtin_amdgcn_wave_barrier();
-    __asm__ volatile("" ::: "memory");  // before the words are reused
 }
 
 // Writes the payload of a wave whose blocks all hold one value, quantized to
@@ -2332,37 +2469,6 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void compress_split_argtable_kernel(
 
 // ---- relative-bound pre-pass (jobs too long for the fused exchange) -------
 
-// Order keys of the 32 fp32 values in d[], as minmax_kernel<1> keeps them: the
-// smallest non-NaN key, and the largest key with kKey32Nan for a NaN.  Read
-// as signed numbers, the patterns with the sign bit clear order by value and
-// lie above all others; read as unsigned numbers, those with the sign bit set
-// lie above all others and order by magnitude (see block_keys): two maxima
-// over the raw words serve a set that holds both signs and no NaN.
-__device__ __forceinline__ void keys32_minmax(const uint32_t* d, uint32_t& kmin,
-                                              uint32_t& kmax) {
-    int32_t smax = INT32_MIN;
-    uint32_t umax = 0;
-#pragma unroll
-    for (int v = 0; v < kBlockElems; ++v) {
-        smax = max(smax, (int32_t)d[v]);
-        umax = max(umax, d[v]);
-    }
-    if (smax >= 0 && smax <= 0x7F800000 && umax >= 0x80000000u && umax <= 0xFF800000u) {
-        kmin = ~umax;
-        kmax = (uint32_t)smax | 0x80000000u;
-        return;
-    }
-    kmin = 0xFFFFFFFFu;
-    kmax = 0u;
-#pragma unroll
-    for (int v = 0; v < kBlockElems; ++v) {
-        const float x = __uint_as_float(d[v]);
-        const uint32_t k = x != x ? kKey32Nan : key32(x);
-        kmax = max(kmax, k);
-        if (x == x) kmin = min(kmin, k);
-    }
-}
-
 // First of the 2048 values of wave `wave` of a tile of a BF16 page when they
 // are all there and lie one behind the other (any 2-byte address); nullptr
 // otherwise (each lane then finds its own block).  Wave-uniform.
@@ -2435,14 +2541,10 @@ __global__ __launch_bounds__(kThreads) void minmax_kernel(MinMaxParams p) {
                     d[4 * i + 2] = v.z;
                     d[4 * i + 3] = v.w;
                 }
-                keys32_minmax(d, kmin, kmax);
+                keys32_minmax(d, kBlockElems, kmin, kmax);
             } else if (count) {
-                // a block's missing values repeat its first one
-                const g_u32* src = to_global(reinterpret_cast<const uint32_t*>(in + e0));
-#pragma unroll
-                for (int v = 0; v < kBlockElems; ++v)
-                    d[v] = src[(uint32_t)v < count ? v : 0];
-                keys32_minmax(d, kmin, kmax);
+                load_block_f32(in, e0, count, d);
+                keys32_minmax(d, count, kmin, kmax);
             }
         } else {
             uint32_t d[16];
@@ -3572,12 +3674,20 @@ hipError_t launch_decompress(const DecompressParams& p, hipStream_t stream,
 
 int compress_resident_workgroups(int device, bool pipelined) {
     int per_cu = 0;
-    const void* fn = pipelined
-        ? reinterpret_cast<const void*>(compress_persistent_kernel<0, true>)
-        : reinterpret_cast<const void*>(compress_kernel<0, 0>);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, fn, pipelined ? kEncThreads : kThreads, 0) != hipSuccess)
-        per_cu = 1;
+    const void* const tile_kernels[3] = {
+        reinterpret_cast<const void*>(compress_kernel<0, 0>),
+        reinterpret_cast<const void*>(compress_kernel<1, 1>),
+        reinterpret_cast<const void*>(compress_lorenzo_kernel<0, kModeOutlier>)};
+    const void* const persistent_kernel =
+        reinterpret_cast<const void*>(compress_persistent_kernel<0, true>);
+    for (int i = 0; i < (pipelined ? 1 : 3); ++i) {
+        int fits = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &fits, pipelined ? persistent_kernel : tile_kernels[i],
+                pipelined ? kEncThreads : kThreads, 0) != hipSuccess)
+            fits = 1;
+        per_cu = i == 0 ? fits : std::min(per_cu, fits);
+    }
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) != hipSuccess) return per_cu;
     return per_cu * prop.multiProcessorCount;
