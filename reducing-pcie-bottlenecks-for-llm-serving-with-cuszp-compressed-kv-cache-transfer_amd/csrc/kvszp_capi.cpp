@@ -461,7 +461,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
             jobs[job].in = reinterpret_cast<const uint16_t*>(in);
             jobs[job].out = reinterpret_cast<uint8_t*>(out);
             jobs[job].eps = e;
-            negative_bound |= e < 0.0f;
+            negative_bound |= bound_is_negative(e);
             jobs[job].reserved = 0;
         }
     }
@@ -1111,7 +1111,7 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
         j.eps = (eps_overrides && eps_overrides[i] > 0.0f) ? eps_overrides[i]
                                                           : c->config.error_bound;
         j.reserved = 0;
-        negative_bound |= j.eps < 0.0f;
+        negative_bound |= bound_is_negative(j.eps);
     }
     // The previous call on this context waited for its kernels, so the
     // staging records are free; the copy goes into the scratch job table.

@@ -31,6 +31,7 @@
 #endif
 
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 namespace kvszp {
@@ -232,6 +233,9 @@ struct Chunk {
 inline bool long_jobs(bool plain_blocks, uint32_t max_tiles_per_job) {
     return plain_blocks && max_tiles_per_job > (uint32_t)kTileBlocks;
 }
+
+// -0.0 is a negative bound: its reciprocal is -inf.
+inline bool bound_is_negative(float eps) { return std::signbit(eps); }
 
 // The launches that the persistent encoder takes: long jobs as above, and jobs
 // of blocks inside one layer whose tiles number at most half its grid (its

@@ -321,6 +321,15 @@ int main() {
         std::printf("first-tile walks=%ld\n", walked);
     }
 
+    // Bounds whose reciprocal is negative stay off the persistent encoder.
+    {
+        const Chunk ch{0, 1, 6, 6, true, false};
+        for (float eps : {1e-4f, 0.0f, 1e-45f, INFINITY})
+            CHECK(persistent_encoder_takes(1536, ch, false, bound_is_negative(eps)), "%g", eps);
+        for (float eps : {-1e-4f, -0.0f, -1e-45f, -INFINITY})
+            CHECK(!persistent_encoder_takes(1536, ch, false, bound_is_negative(eps)), "%g", eps);
+    }
+
     std::printf("launches=%ld tiles=%ld mismatches=%ld\n", launches, tiles_checked, g_bad);
     return g_bad == 0 ? 0 : 1;
 }

@@ -43,11 +43,13 @@ def check(oracle, pages, n, eps, relative, bufs, sizes, bounds):
 
 
 # bound: relative, absolute, absolute with an infinite reciprocal, negative
+# (-0.0: its reciprocal is -inf)
 @pytest.mark.parametrize("eps,relative", [(1e-4, True), (1e-3, False), (1e-40, False),
-                                          (-1e-2, False), (-1e-4, True)])
+                                          (-1e-2, False), (-1e-4, True), (-0.0, False),
+                                          (-0.0, True)])
 @pytest.mark.parametrize("n,off", [(1, 1), (31, 0), (33, 3), (2047, 1), (2049, 0), (4095, 5),
                                    (4097, 1), (6145, 0), (8191, 7), (8193, 1),
-                                   (5 * 8192 + 4096, 1), (30 * 8192 + 2080 + 17, 3)])
+                                   (5 * 8192 + 4096, 0), (5 * 8192 + 4096, 1), (30 * 8192 + 2080 + 17, 3)])
 def test_cut_blocks(oracle, n, off, eps, relative):
     import cuszp_wrapper_cpp as cpp
 
