@@ -652,7 +652,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
     }
     if (__atomic_load_n(&c->host_ctl[kHostOverflow], __ATOMIC_ACQUIRE) == seq) {
         // Jobs whose staged payload overflowed in the persistent encoder
-        // (rates near 31 throughout): those jobs again, one workgroup per tile.
+        // (mean rates above 24): those jobs again, one workgroup per tile.
         std::vector<const void*> in;
         std::vector<void*> out;
         std::vector<uint64_t> cap;

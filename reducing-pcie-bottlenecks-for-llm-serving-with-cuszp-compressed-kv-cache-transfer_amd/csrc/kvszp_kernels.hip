@@ -1812,7 +1812,13 @@ __device__ __forceinline__ void pending_results(const CompressParams& p, const P
 // per wave.
 constexpr int kEncThreads = 128;
 constexpr int kEncWaves = kEncThreads / 64;
-constexpr int kEncStageWords = 2 * 64 * 16 + 16;  // 128 blocks of <= 16 words
+// A wave's staging words: 128 blocks of 25 words (a mean rate of 24), the most
+// that leaves room for six workgroups in a compute unit's 160 KiB.  A wave
+// with more marks its job for a second encode.  With 16 words per block, the
+// bounds that give rates of 16 to 24 paid for both encodes: two segments of
+// 32 Mi values at an absolute 1e-5 382 us, now 121 (with one workgroup per tile
+// 174); one segment of 100003 values 67 us, now 37 (40).
+constexpr int kEncStageWords = 2 * 64 * 25 + 16;
 
 // Launches whose jobs have at most this many tiles run the persistent
 // encoder that does the look-back of the staged tile beside the bound
@@ -2296,8 +2302,8 @@ __device__ __forceinline__ void compress_persistent(const CompressParams& p) {
         // the exact quantizer's low fields ((|q| << 1) | sign) & 0xFFFF,
         // whose transpose gives words 0..15 in stream order, and for rates
         // above 15 the high fields |q| >> 15 (words 16..31), staged exactly.
-        // A wave whose payload would not fit the staging words (rates far
-        // above 15 throughout) stages nothing.  When all its blocks hold one
+        // A wave whose payload would not fit the staging words (a mean rate
+        // above 24) stages nothing.  When all its blocks hold one
         // value (every block's min and max keys are the same key: no NaN, no
         // absent block), as on a constant page under a relative bound, its
         // payload is that value's block repeated, written at d. from q alone.
