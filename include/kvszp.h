@@ -345,7 +345,9 @@ int kvszp_reencode_count(const kvszp_ctx* ctx, uint64_t* count);
  * staging overflow (as kvszp_reencode_count), and compress calls that ran
  * the schedule needing no residency from the start because a launch of the
  * context gave up within the previous KVSZP_SAFE_CALLS calls (default 0:
- * every call tries the persistent encoder).  No reference counterpart. */
+ * every call tries the persistent encoder), or, for segments of more than
+ * 256 tiles of 8192 values, within the previous 64 calls of such segments.
+ * No reference counterpart. */
 int kvszp_schedule_counts(const kvszp_ctx* ctx, uint64_t* reencoded, uint64_t* safe_calls);
 
 /* Sets the time bound of the encoders' cross-workgroup waits of this

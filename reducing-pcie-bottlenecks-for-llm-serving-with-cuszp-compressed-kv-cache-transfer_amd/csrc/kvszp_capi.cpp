@@ -104,6 +104,14 @@ struct kvszp_ctx {
     // too.  `safe_left` counts them down.
     uint32_t safe_after_abort = 0;
     uint32_t safe_left = 0;
+    // The same for calls of long jobs (long_jobs), always: their tiles wait for
+    // every earlier one of the grid's round, so beside a kernel that holds
+    // compute units until all its own workgroups have run, each such launch
+    // gives up, whatever its bound.  Two segments of 32 Mi values beside three
+    // products of 8192 x 8192 matrices: 2630 us a call when every call tries,
+    // 1680 us on average over 65 calls with this (1645 without the one that
+    // tries); on an idle device 107 us, and 149 in the calls after a give-up.
+    uint32_t long_safe_left = 0;
     uint64_t safe_calls = 0;      // compress calls run on that schedule
     // Epoch tags run from 1 to epoch_limit, then every tagged word is
     // cleared and they start again (KVSZP_EPOCH_LIMIT lowers the limit so
@@ -292,6 +300,23 @@ int next_epoch(kvszp_ctx* c, hipStream_t stream, uint32_t* epoch) {
     }
     *epoch = ++c->epoch;
     return KVSZP_OK;
+}
+
+constexpr uint32_t kLongSafeCalls = 64;
+
+// True when a call of long jobs is to run without the persistent encoder, as a
+// recent one gave up; counted down once per call.
+bool skip_long_encoder(kvszp_ctx* c, bool long_call) {
+    if (!long_call || c->long_safe_left == 0) return false;
+    c->long_safe_left -= 1;
+    c->safe_calls += 1;
+    return true;
+}
+
+// A launch of the call gave up (`long_call`: on the persistent encoder for long jobs).
+void note_give_up(kvszp_ctx* c, bool long_call) {
+    c->safe_left = c->safe_after_abort;
+    if (long_call) c->long_safe_left = kLongSafeCalls;
 }
 
 int check_fixed_config(const kvszp_ctx* c) {
@@ -511,6 +536,11 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
     // needs no residency (pre-pass bound, one workgroup per tile, untimed
     // look-back on earlier workgroups); otherwise the fused bound and the
     // persistent encoder where they apply, with time-bounded waits.
+    bool long_call = false;  // a chunk for the persistent encoder for long jobs
+    for (const Chunk& ch : chunks)
+        long_call |= !f32 && long_jobs(ch.plain_blocks, ch.max_tiles_per_job) &&
+                     c->pipelined_grid != 0 && !negative_bound;
+    bool skip_long = false;
     std::vector<char> redo_candidate(chunks.size(), 0);
     std::vector<size_t> chunk_first_job(chunks.size(), 0);
     for (size_t k = 1; k < chunks.size(); ++k) {
@@ -529,11 +559,11 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
             bound_mode = (!safe && ch.max_tiles_per_job <= c->fused_tile_limit)
                              ? kBoundFused : kBoundPrepass;
         const bool prepass = bound_mode == kBoundPrepass;
+        const bool lng = long_jobs(ch.plain_blocks, ch.max_tiles_per_job);
         const bool persistent =
-            !safe && !f32 &&
+            !safe && !f32 && !(lng && skip_long) &&
             persistent_encoder_takes(c->pipelined_grid, ch, prepass, negative_bound);
-        const bool use_arg = persistent && arg_table &&
-                             !long_jobs(ch.plain_blocks, ch.max_tiles_per_job);
+        const bool use_arg = persistent && arg_table && !lng;
         if (!use_arg) {
             const int r = need_table();
             if (r) return r;
@@ -626,6 +656,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         c->safe_calls += 1;
         schedule_safe = true;
     }
+    skip_long = skip_long_encoder(c, long_call && !schedule_safe);
     for (size_t k = 0; k < chunks.size(); ++k)
         if ((rc = launch_chunk(k, schedule_safe, true))) return rc;
 
@@ -642,7 +673,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         e = wait_stream(stream);
         if (e != hipSuccess) return hip_fail(e, "waiting for the encoder");
         c->redone += 1;
-        c->safe_left = c->safe_after_abort;
+        note_give_up(c, long_call);
     }
     rc = consume_device_error(c, stream);
     if (rc) return rc;
@@ -1199,9 +1230,11 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
     p.quantizer = c->quantizer;
     p.aligned16 = aligned16 ? 1 : 0;
     const Chunk chunk{0, 1, p.total_tiles, tiles_per_job, true, n % kBlockElems == 0};
-    const bool persistent =
-        !schedule_safe && persistent_encoder_takes(c->pipelined_grid, chunk,
-                                                   bound_mode == kBoundPrepass, negative_bound);
+    const bool takes = !schedule_safe &&
+                       persistent_encoder_takes(c->pipelined_grid, chunk,
+                                                bound_mode == kBoundPrepass, negative_bound);
+    const bool long_call = takes && long_jobs(chunk.plain_blocks, tiles_per_job);
+    const bool persistent = takes && !skip_long_encoder(c, long_call);
     if (persistent || bound_mode == kBoundFused) {
         p.abort_word = words + kScratchAbort / 8;
         p.wait_ticks = c->wait_ticks;
@@ -1217,7 +1250,7 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
     if (e != hipSuccess) return hip_fail(e, "waiting for the encoder");
     const bool gave_up = p.abort_word != nullptr &&
                          __atomic_load_n(&c->host_ctl[kHostAbort], __ATOMIC_ACQUIRE) == seq;
-    if (gave_up) c->safe_left = c->safe_after_abort;
+    if (gave_up) note_give_up(c, long_call);
     if (p.abort_word != nullptr &&
         (gave_up || __atomic_load_n(&c->host_ctl[kHostOverflow], __ATOMIC_ACQUIRE) == seq)) {
         // Staging overflow, or a bounded wait gave up: the schedule that
