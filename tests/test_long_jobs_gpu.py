@@ -72,9 +72,18 @@ def test_overflow_and_uniform(oracle):
     assert w._ctx.reencode_count() == before + 1
 
 
-# A job of 900 tiles may meet every look-back's words at the first poll, even
-# with a wait bound of zero; over the rounds of this many, some poll again.
-MANY = 4096 * 8192
+MANY = 4096 * 8192   # 8192 tiles in two jobs: more than five rounds of the grid
+
+
+def until_give_up(ctx, call):
+    """Calls until a launch gives up: with a wait bound of zero the first wait
+    that is not met at its first poll does, which any of thousands can be."""
+    before = ctx.reencode_count()
+    for _ in range(5):
+        call()
+        if ctx.reencode_count() > before:
+            break
+    assert ctx.reencode_count() == before + 1
 
 
 def test_give_up(oracle):
@@ -83,8 +92,8 @@ def test_give_up(oracle):
     store_and_check(oracle, w, pages_of(2, 900 * 8192), 1e-4, True, 0)
     w = wrapper(True)
     w._ctx.set_wait_bound(0)
-    store_and_check(oracle, w, pages_of(2, MANY), 1e-4, True, 0)
-    assert w._ctx.reencode_count() == 1
+    pages = pages_of(2, MANY)
+    until_give_up(w._ctx, lambda: store_and_check(oracle, w, pages, 1e-4, True, 0))
 
 
 AFTER = 64  # long calls after a give-up that stay off the persistent encoder
@@ -94,19 +103,24 @@ def test_calls_after_a_give_up(oracle):
     w = wrapper(True)
     w._ctx.set_wait_bound(0)
     pages = pages_of(2, MANY)
+    bufs = [torch.empty(8 * pages.shape[1], dtype=torch.uint8, device="cuda") for _ in range(2)]
+
+    def store():
+        assert w.compress_batch_fixed_bf16(list(pages), bufs, [1e-4] * 2)[0]
+
     counts = w._ctx.schedule_counts
-    store_and_check(oracle, w, pages, 1e-4, True, 0)
+    until_give_up(w._ctx, store)
     assert counts() == {"reencoded": 1, "safe_calls": 0}
     store_and_check(oracle, w, pages, 1e-4, True, 0)
     assert counts() == {"reencoded": 1, "safe_calls": 1}
-    store_and_check(oracle, w, pages_of(40, 9 * 8192), 1e-4, True, 0)  # shorter jobs try on
-    assert counts() == {"reencoded": 2, "safe_calls": 1}
-    bufs = [torch.empty(8 * pages.shape[1], dtype=torch.uint8, device="cuda") for _ in range(2)]
+    store_and_check(oracle, w, pages_of(40, 9 * 8192), 1e-4, True, 0)  # shorter jobs do not count
+    assert counts()["safe_calls"] == 1
+    before = w._ctx.reencode_count()
     for _ in range(AFTER - 1):
-        assert w.compress_batch_fixed_bf16(list(pages), bufs, [1e-4] * 2)[0]
-    assert counts() == {"reencoded": 2, "safe_calls": AFTER}
-    store_and_check(oracle, w, pages, 1e-4, True, 0)
-    assert counts() == {"reencoded": 3, "safe_calls": AFTER}
+        store()
+    assert counts() == {"reencoded": before, "safe_calls": AFTER}
+    until_give_up(w._ctx, store)
+    assert counts()["safe_calls"] == AFTER
 
 
 def test_no_allocation_calls_after_a_give_up(oracle):
@@ -124,14 +138,19 @@ def test_no_allocation_calls_after_a_give_up(oracle):
     host = bits(pages)
     want = [oracle.compress_page(host[i], n, float(oracle.relative_bound(host[i], n, 1e-4)))
             for i in range(2)]
-    for safe in (0, 1, 2):
+
+    def store():
         for b in bufs:
             b.fill_(0xAB)
         kvszp.check(ctx.compress_noalloc(
             kvszp.ptr_array([p.data_ptr() for p in pages]),
             kvszp.ptr_array([b.data_ptr() for b in bufs]), kvszp.u64_array([8 * n] * 2), None,
             2, n, torch.cuda.current_stream().cuda_stream, sizes, bounds))
-        assert ctx.schedule_counts() == {"reencoded": 1, "safe_calls": safe}
         for i in range(2):
             assert sizes[i] == len(want[i])
             assert np.array_equal(bufs[i][:sizes[i]].cpu().numpy(), want[i])
+
+    until_give_up(ctx, store)
+    for safe in (1, 2):
+        store()
+        assert ctx.schedule_counts() == {"reencoded": 1, "safe_calls": safe}
