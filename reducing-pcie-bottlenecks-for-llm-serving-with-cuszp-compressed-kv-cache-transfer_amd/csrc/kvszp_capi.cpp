@@ -498,7 +498,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
             return fail(KVSZP_EINVAL, "batch too large for one launch");
         max_tiles = std::max(max_tiles, ch.tiles);
         minmax_words = std::max(minmax_words, batch * minmax_stride(minmax_shards(
-                                    ch.tiles, ch.max_tiles_per_job, batch, UINT64_MAX)));
+                                    ch.tiles, ch.max_tiles_per_job, batch, kMinMaxWords)));
     }
 
     const bool relative = c->config.use_relative_error != 0 && !bounds_given;
@@ -553,7 +553,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         CompressParams p;
         std::memset(&p, 0, sizeof(p));
         p.num_groups = fill_groups(p.groups, specs, ch, chunk_first_job[k]);
-        p.minmax_shards = minmax_shards(ch.tiles, ch.max_tiles_per_job, batch, UINT64_MAX);
+        p.minmax_shards = minmax_shards(ch.tiles, ch.max_tiles_per_job, batch, kMinMaxWords);
         int bound_mode = kBoundAbsolute;
         if (relative)
             bound_mode = (!safe && ch.max_tiles_per_job <= c->fused_tile_limit)

@@ -150,6 +150,10 @@ constexpr uint32_t kMinMaxTilesPerWg = 4;
 // job with one shard takes just its pair.
 constexpr uint32_t kMinMaxShardWords = 8;
 constexpr uint32_t kMinMaxShards = 32;
+// Words of a context's launch at most (8 MiB: 32 shards for 4096 jobs), or a
+// pair per job: the shards follow the launch's longest job, and one of those
+// beside 100 000 short ones asked for 205 MB.
+constexpr uint64_t kMinMaxWords = 1ull << 20;
 
 KVSZP_PLAN_FN uint32_t minmax_tiles_per_wg(uint64_t tiles) {
     const uint64_t per = tiles / kMinMaxWorkgroups;

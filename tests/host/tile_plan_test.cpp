@@ -48,6 +48,43 @@ static void check_runs(const std::vector<uint32_t>& starts, uint32_t total, cons
               starts[b - 1], total);
 }
 
+// The pre-pass of a launch: its workgroups' publications (a job's words of the
+// workgroup's shard, whenever the job or the workgroup ends) stay inside the
+// job's words and those inside `words`, and every job gets one.
+static void check_prepass(const std::vector<GroupSpec>& specs, const Chunk& ch,
+                          size_t first_job, size_t batch, uint64_t words) {
+    Group groups[kMaxGroups];
+    const int ng = fill_groups(groups, specs, ch, first_job);
+    uint32_t first_tiles[kMaxGroups];
+    for (int i = 0; i < ng; ++i) first_tiles[i] = groups[i].first_tile;
+    const uint32_t total = (uint32_t)ch.tiles;
+    const uint32_t per = minmax_tiles_per_wg(total);
+    CHECK(per >= 1 && per <= kMinMaxTilesPerWg, "%u tiles per workgroup", per);
+    CHECK(per == 1 || total / per >= kMinMaxWorkgroups, "%u tiles in workgroups of %u", total, per);
+    const uint32_t shards = minmax_shards(total, ch.max_tiles_per_job, batch, words);
+    const uint64_t stride = minmax_stride(shards);
+    CHECK(shards >= 1 && shards <= kMinMaxShards && (shards & (shards - 1)) == 0, "%u shards", shards);
+    CHECK(batch * stride <= std::max<uint64_t>(words, 2 * batch), "%zu jobs x %llu words", batch,
+          (unsigned long long)stride);
+    std::vector<uint8_t> met(batch, 0);
+    for (uint32_t t0 = 0; t0 < total; t0 += per) {
+        const uint32_t end = std::min(t0 + per, total);
+        for (uint32_t t = t0; t < end;) {
+            const TilePlace pl = place_tile(groups, first_tiles, ng, t);
+            ++t;
+            if (t < end && pl.tile + 1 < groups[pl.gi].tiles_per_job) continue;
+            const uint64_t at = (uint64_t)((pl.tile / per) & (shards - 1)) * kMinMaxShardWords;
+            CHECK(at + 2 <= stride, "tile %u of a job: word %llu of %llu", pl.tile,
+                  (unsigned long long)at, (unsigned long long)stride);
+            CHECK(pl.job < batch, "job %u of %zu", pl.job, batch);
+            if (pl.job < batch) met[pl.job] = 1;
+        }
+    }
+    size_t jobs = 0;
+    for (size_t gi = ch.g0; gi < ch.g1; ++gi) jobs += specs[gi].jobs;
+    for (size_t j = first_job; j < first_job + jobs; ++j) CHECK(met[j], "job %zu has no word", j);
+}
+
 // One launch: placement, plan checks, decoder runs.
 static void check_launch(const std::vector<GroupSpec>& specs, const Chunk& ch,
                          size_t first_job, const std::vector<uint64_t>& sizes,
@@ -206,6 +243,8 @@ int main() {
         for (const Chunk& ch : chunks) {
             CHECK(ch.g1 - ch.g0 <= (size_t)kMaxGroups && ch.g1 > ch.g0, "chunk groups");
             check_launch(specs, ch, first_job, sizes, &tiles_checked);
+            for (uint64_t words : {kMinMaxWords, (uint64_t)8192, (uint64_t)0})
+                check_prepass(specs, ch, first_job, batch, words);
             for (size_t gi = ch.g0; gi < ch.g1; ++gi) first_job += specs[gi].jobs;
             ++launches;
         }
@@ -319,6 +358,50 @@ int main() {
         CHECK(persistent_slot_cus(229376, 1500, 256, 1) == 0, "grid not a multiple of the units");
         CHECK(persistent_slot_cus(229376, 256, 256, 1) == 0, "one workgroup per unit");
         std::printf("first-tile walks=%ld\n", walked);
+    }
+
+    // The pre-pass at the sizes that take several tiles per workgroup and
+    // several shards, and the words' limits: a long job beside many short ones,
+    // and the no-allocation entry's fixed array (2 words for each of 4096 jobs).
+    {
+        for (const std::vector<GroupSpec>& specs :
+             {std::vector<GroupSpec>{GroupSpec{257 * 8192, nullptr, 0, 0, 0, 16}},
+              std::vector<GroupSpec>{GroupSpec{4096 * 8192, nullptr, 0, 0, 0, 2}},
+              std::vector<GroupSpec>{GroupSpec{1100 * 8192 + 5, nullptr, 0, 0, 0, 7},
+                                     GroupSpec{8192 * 3, nullptr, 0, 0, 0, 700}},
+              std::vector<GroupSpec>{GroupSpec{1100 * 8192, nullptr, 0, 0, 0, 1},
+                                     GroupSpec{32, nullptr, 0, 0, 0, 100000}}}) {
+            const std::vector<Chunk> chunks = split_chunks(specs);
+            size_t batch = 0;
+            for (const GroupSpec& s : specs) batch += s.jobs;
+            for (uint64_t words : {kMinMaxWords, (uint64_t)8192})
+                check_prepass(specs, chunks[0], 0, batch, words);
+        }
+        CHECK(minmax_shards(8192, 4096, 2, kMinMaxWords) == 32, "two segments of 32 Mi values");
+        CHECK(minmax_shards(104096, 1100, 100001, kMinMaxWords) == 1, "words past the limit");
+        CHECK(minmax_shards(65536, 16, 4096, 8192) == 1, "no-allocation entry, 4096 jobs");
+        CHECK(minmax_shards(65536, 32768, 2, 8192) == 32, "no-allocation entry, 2 jobs");
+    }
+
+    // The launches of the persistent encoder: blocks of one layer with at most
+    // half a grid of tiles per job and the bound not from the pre-pass, and
+    // long jobs (whole blocks, no layer map) whatever their bound's source.
+    {
+        const uint32_t G = 1536;
+        for (uint32_t tpj : {1u, 256u, 257u, 768u, 769u, 65536u})
+            for (bool one_layer : {false, true})
+                for (bool plain : {false, true})
+                    for (bool prepass : {false, true}) {
+                        const Chunk ch{0, 1, tpj, tpj, one_layer, plain};
+                        const bool lng = plain && tpj > 256;
+                        CHECK(long_jobs(plain, tpj) == lng, "%u tiles", tpj);
+                        const bool takes = persistent_encoder_takes(G, ch, prepass, false);
+                        CHECK(takes == (lng || (!prepass && one_layer && tpj <= G / 2)),
+                              "%u tiles, one layer %d, plain %d, pre-pass %d", tpj, one_layer,
+                              plain, prepass);
+                        CHECK(!persistent_encoder_takes(0, ch, prepass, false), "no grid");
+                        CHECK(!persistent_encoder_takes(G, ch, prepass, true), "negative bound");
+                    }
     }
 
     // Bounds whose reciprocal is negative stay off the persistent encoder.
