@@ -1,8 +1,9 @@
 """The relative-bound pre-pass over segments of every shape it meets: BF16
-segments past the in-kernel exchange (more than 256 tiles) and fp32 pages,
-which always take it.  The extremes sit where a wave's wide loads end (a
-partial last run or block) and at addresses that are only 2- or 4-byte
-aligned.  Bounds and streams against the oracle."""
+segments and fp32 pages of more than 256 tiles (up to there the bound is
+exchanged inside the encoder, as in test_fp32_pages), in workgroups of one and
+of several tiles.  The extremes sit where a wave's wide loads end (a partial
+last run or block), at the ends of neighbouring jobs, and at addresses that are
+only 2- or 4-byte aligned.  Bounds and streams against the oracle."""
 
 from __future__ import annotations
 
@@ -71,6 +72,56 @@ def test_long_bf16_runs_across_layers(oracle):
         assert np.float32(bounds[i]) == np.float32(eb)
         want = oracle.compress_page(host[i], n, float(eb), idx, src, epl)
         assert np.array_equal(bufs[i][:sizes[i]].cpu().numpy(), want)
+
+
+# 4112 tiles: two per workgroup, up to 16 shards a job; 8198: four and 32.
+# Whole blocks run on the persistent encoder for long jobs, cut ones do not.
+@pytest.mark.parametrize("count,n,off", [(16, LONG + 8192, 0), (16, LONG + 4096 + 17, 1),
+                                         (2, 4099 * 8192, 0)])
+def test_several_tiles_per_workgroup(oracle, count, n, off):
+    pages = flat_pages(count, n, off, torch.bfloat16, count)
+    for i in range(count):   # each job's own extremes, next to its neighbours'
+        pages[i, 0], pages[i, -1] = 10.0 + i, -20.0 - 3 * i
+    w = fixed_wrapper()
+    bufs = [buffer(n) for _ in range(count)]
+    ok, sizes, bounds = w.compress_batch_fixed_bf16(list(pages), bufs, [1e-4] * count)
+    assert ok
+    host = bits(pages)
+    want, _, want_bounds = oracle.compress_batch(host, [1e-4] * count, relative=True, threads=8)
+    for i in range(count):
+        assert np.float32(bounds[i]) == np.float32(want_bounds[i]), i
+        assert np.array_equal(bufs[i][:sizes[i]].cpu().numpy(), want[i]), i
+
+
+@pytest.mark.parametrize("mode", ["fixed", "plain", "outlier"])
+@pytest.mark.parametrize("n,off", [(LONG + 2048 + 33, 3), (LONG + 2047, 0), (300 * 8192, 1)])
+def test_long_fp32_pages(oracle, mode, n, off):
+    import cuszp_wrapper_cpp as cpp
+
+    m = {"fixed": cpp.MODE_FIXED, "plain": cpp.MODE_PLAIN, "outlier": cpp.MODE_OUTLIER}[mode]
+    w = cpp.CuSZpWrapper(cpp.CompressionConfig(1e-4, True, cpp.DIM_1D, m, cpp.TYPE_FLOAT), 0)
+    kinds = 6
+    pages = flat_pages(kinds, n, off, torch.float32, n)
+    pages[0, 0], pages[0, -1] = -9.0, 7.0
+    pages[1] = pages[1].abs() + 0.5
+    pages[2] = -pages[2].abs()
+    pages[2, -1] = -60.0
+    pages[3] = 0.0
+    pages[3, -1] = -0.0
+    pages[4, -1] = float("nan")
+    pages[5, 0], pages[5, -1] = float("inf"), -3.0
+    host = pages.cpu().numpy()
+    for i in range(kinds):
+        buf = torch.full((8 * n + 1024 + 136,), 0xAB, dtype=torch.uint8, device="cuda")
+        ok, buf, size, bound = w.compress(pages[i], buf, 1e-4)
+        assert ok
+        eb = np.float32(oracle.relative_bound_f32(host[i], 1e-4))
+        assert np.float32(bound) == eb or (np.isnan(eb) and np.isnan(bound)), i
+        want = (oracle.compress_page_f32(host[i], float(eb)) if mode == "fixed"
+                else oracle.compress_page_f32_mode(host[i], float(eb), int(m)))
+        assert size == want.size, i
+        assert np.array_equal(buf[:size].cpu().numpy(), want), i
+        assert bool((buf[size:] == 0xAB).all()), i
 
 
 @pytest.mark.parametrize("n", [1, 31, 2047, 2048, 8193, 5 * 8192 + 33])
