@@ -73,8 +73,11 @@ def test_batches(oracle, n, give_up):
         w._ctx.set_wait_bound(0)
     pages = pages_of(n, 0)[:3]
     bufs = [torch.empty(8 * n, dtype=torch.uint8, device="cuda") for _ in range(3)]
+    before = w._ctx.reencode_count()
     ok, sizes, bounds = w.compress_batch_fixed(list(pages), bufs, [1e-4, 1e-3, 1e-5])
     assert ok
+    # past 256 tiles the pre-pass gives the bound and no wait is timed
+    assert w._ctx.reencode_count() - before == (1 if give_up and n <= 256 * 8192 else 0)
     for i, eps in enumerate((1e-4, 1e-3, 1e-5)):
         x = pages[i].cpu().numpy()
         eb = oracle.relative_bound_f32(x, eps)
