@@ -3717,16 +3717,20 @@ hipError_t launch_decompress(const DecompressParams& p, hipStream_t stream,
 
 int compress_resident_workgroups(int device, bool pipelined) {
     int per_cu = 0;
-    const void* const tile_kernels[3] = {
+    const void* const tile_kernels[4] = {
         reinterpret_cast<const void*>(compress_kernel<0, 0>),
         reinterpret_cast<const void*>(compress_kernel<1, 1>),
+        reinterpret_cast<const void*>(compress_lorenzo_kernel<0, kModePlain>),
         reinterpret_cast<const void*>(compress_lorenzo_kernel<0, kModeOutlier>)};
-    const void* const persistent_kernel =
-        reinterpret_cast<const void*>(compress_persistent_kernel<0, true>);
-    for (int i = 0; i < (pipelined ? 1 : 3); ++i) {
+    const void* const persistent_kernels[4] = {
+        reinterpret_cast<const void*>(compress_persistent_kernel<0, true>),
+        reinterpret_cast<const void*>(compress_cut_kernel<0, true>),
+        reinterpret_cast<const void*>(compress_split_kernel<0, true>),
+        reinterpret_cast<const void*>(compress_long_kernel<0>)};
+    for (int i = 0; i < 4; ++i) {
         int fits = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &fits, pipelined ? persistent_kernel : tile_kernels[i],
+                &fits, pipelined ? persistent_kernels[i] : tile_kernels[i],
                 pipelined ? kEncThreads : kThreads, 0) != hipSuccess)
             fits = 1;
         per_cu = i == 0 ? fits : std::min(per_cu, fits);

@@ -11,8 +11,8 @@ SGPR file allows on MI355X.  Measured with a probe kernel of 256 threads,
 says 8); 96 -> 6 (the query says 7); with 80 VGPRs, 100 -> 6.  So each
 kernel's SGPR count is held to what its target occupancy allows:
   * decoder: 8 waves per SIMD (64 VGPRs) and next_free_sgpr <= 74;
-  * encoder: two-wave workgroups at 3 waves per SIMD (168 VGPRs, six
-    workgroups per CU) and next_free_sgpr <= 100 (3 x 100 SGPRs per SIMD is
+  * encoder, in each of its kinds: two-wave workgroups at 3 waves per SIMD
+    (168 VGPRs, six workgroups per CU) and next_free_sgpr <= 100 (3 x 100 SGPRs per SIMD is
     far below the limit measured above); six workgroups' LDS must fit the
     CU's 160 KiB.
 """
@@ -58,6 +58,8 @@ def kernels(tmp_path_factory):
         }
     # explicit (by_value) arguments of each kernel: (offset, size)
     notes = text[text.index("amdhsa.kernels:"):]
+    for m in re.finditer(r"\.max_flat_workgroup_size: (\d+)\n\s+\.name:\s+(\S+)", notes):
+        meta[m.group(2)]["threads"] = int(m.group(1))
     for m in re.finditer(r"  - \.agpr_count:.*?\.args:\n(.*?)\n    \.[a-z_]+:.*?\.name:\s+(\S+)",
                          notes, re.S):
         if m.group(2) in meta:
@@ -83,15 +85,29 @@ def test_persistent_decoder_fits_eight_waves(kernels):
         assert m["scratch"] == 0, (k, m)
 
 
-def test_persistent_encoder_fits_three_waves(kernels):
-    for k, m in {**pick(kernels, "compress_persistent_kernel"),
-                 **pick(kernels, "compress_persistent_argtable_kernel")}.items():
-        if "decompress" in k:
-            continue
+# Kernels of each kind of persistent encoder launch: by quantizer and (long
+# jobs excepted) look-back placement, with and without an argument table.
+ENCODERS = {"persistent": 4, "cut": 4, "split": 4, "long": 2}
+LDS_UNIT = 1280  # LDS is allocated in 1/128ths of the 160 KiB
+
+
+@pytest.mark.parametrize("kind", list(ENCODERS))
+def test_persistent_encoder_fits_three_waves(kernels, kind):
+    got = {k: m for k, m in kernels.items()
+           if f"compress_{kind}_" in k and "decompress" not in k}
+    assert len(got) == ENCODERS[kind] * (1 if kind == "long" else 2), sorted(got)
+    for k, m in got.items():
         assert m["vgpr"] <= 168, (k, m)
         assert m["sgpr"] <= 100, (k, m)
-        assert 6 * m["lds"] <= 160 * 1024, (k, m)
+        assert 6 * -(-m["lds"] // LDS_UNIT) * LDS_UNIT <= 160 * 1024, (k, m)
         assert m["scratch"] == 0, (k, m)
+
+
+def test_every_two_wave_encoder_is_budgeted(kernels):
+    """A kind that is not in ENCODERS has no budget: kernels are told by the
+    128-thread launch bound that only the persistent encoder has."""
+    named = sum(n * (1 if kind == "long" else 2) for kind, n in ENCODERS.items())
+    assert sum(m["threads"] == 128 for m in kernels.values()) == named
 
 
 def test_arg_table_layout(kernels):
@@ -100,9 +116,8 @@ def test_arg_table_layout(kernels):
     compiler must place the second argument exactly there, with the size
     the host copies (kArgTableBytes), and the whole argument segment must
     stay within what the runtime was measured to carry (16 648 bytes)."""
-    got = {**pick(kernels, "compress_persistent_argtable_kernel"),
-           **pick(kernels, "decompress_persistent_argtable_kernel")}
-    assert len(got) == 7  # 4 encoder and 3 decoder instantiations
+    got = pick(kernels, "argtable_kernel")
+    assert len(got) == 15  # 4 of each encoder kind but the long one, 3 decoders
     for k, m in got.items():
         (o0, z0), (o1, z1) = m["args"]
         assert o0 == 0 and o1 == (z0 + 15) // 16 * 16, (k, m["args"])
