@@ -1414,8 +1414,8 @@ __global__ __launch_bounds__(kThreads) void compress_lorenzo_kernel(CompressPara
 // multiple of 32 values; segments without a layer map may have any length and
 // pages any 2-byte address).  Workgroup w encodes
 // tiles w, w + G, w + 2G, ... (G = gridDim.x, at most the number of
-// co-resident workgroups), one 32-value block per thread held in registers
-// together with the block's min/max keys.  Per tile t:
+// co-resident workgroups), two 32-value blocks per thread held in registers
+// together with the blocks' min/max keys.  Per tile t:
 //   a. exchange: min/max over all tiles of t's job -> bound, reciprocal
 //   b. rates: while every |x * recip| of a block stays below 2^30 and the block
 //      holds no NaN, the quantizer (cu:10-25) is monotone in x, so the
@@ -1434,7 +1434,8 @@ __global__ __launch_bounds__(kThreads) void compress_lorenzo_kernel(CompressPara
 // once a job has at most G/2 tiles (a publish that depends on a wait is the
 // min/max of tile u + G, behind the look-back of u; tiles u + G and u are in
 // different jobs), so with all G workgroups resident no cycle of waits
-// exists.  All waits are bounded.
+// exists.  Longer jobs have no exchange (kEncLong) or a bound that needs none:
+// their look-backs alone always reach an earlier tile.  All waits are bounded.
 
 // threadIdx.x behind an empty asm: values derived from it inside the tile
 // loop are recomputed each iteration instead of being hoisted out of the
@@ -1951,8 +1952,9 @@ __device__ __forceinline__ void stage_high_words(const uint32_t* P, uint32_t cou
 // waits that poll again) out of the loop's code: its two copies of the
 // iteration share 64 KiB of instruction cache between two compute units, and
 // with the rare paths in between, a launch's time followed the kernel's place
-// in the code object (2048 blocks of 458752 values: the same instructions 657
-// or 666 us; with the hints 650).
+// in the code object.  Medians of two processes each, without and with the
+// hints: 2048 blocks of 458752 values 658 and 661, 648 and 649 us; 256 blocks of
+// 229376 values 53.6 and 53.0, 51.9 and 51.6.
 //
 // Per tile: the next tile starts loading; (c) its keys; (a) wave 0 gathers
 // the job's min/max and works out the bound while wave 1 finishes the
@@ -2483,7 +2485,7 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void compress_split_argtable_kernel(
     compress_persistent<kQuant, kEarly, kEncSplit>(p);
 }
 
-// ---- relative-bound pre-pass (jobs too long for the fused exchange) -------
+// ---- relative-bound pre-pass (jobs too long for the exchange, re-encodes) --
 
 // First of the 2048 values of wave `wave` of a tile of a BF16 page when they
 // are all there and lie one behind the other (any 2-byte address); nullptr
