@@ -342,12 +342,11 @@ int kvszp_timing_durations(kvszp_ctx* ctx, int kind, double* ms_out,
 int kvszp_reencode_count(const kvszp_ctx* ctx, uint64_t* count);
 
 /* Compress calls of this context encoded again after a give-up or a
- * staging overflow (as kvszp_reencode_count), and compress calls that ran
- * the schedule needing no residency from the start because a launch of the
- * context gave up within the previous KVSZP_SAFE_CALLS calls (default 0:
- * every call tries the persistent encoder), or, for segments of more than
- * 256 tiles of 8192 values, within the previous 64 calls of such segments.
- * No reference counterpart. */
+ * staging overflow (as kvszp_reencode_count), and compress calls kept off the
+ * persistent encoder because launches of the context gave up: the 64 calls
+ * after three give-ups in a row, of at least as many tiles, or, where
+ * KVSZP_SAFE_CALLS is set, that many calls after each give-up, on the schedule
+ * needing no residency.  No reference counterpart. */
 int kvszp_schedule_counts(const kvszp_ctx* ctx, uint64_t* reencoded, uint64_t* safe_calls);
 
 /* Sets the time bound of the encoders' cross-workgroup waits of this

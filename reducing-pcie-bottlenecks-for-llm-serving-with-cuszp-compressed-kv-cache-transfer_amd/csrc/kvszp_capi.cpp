@@ -100,18 +100,20 @@ struct kvszp_ctx {
     // default 0: off).  Measured on MI355X beside a stream of large matrix
     // products, the persistent encoder did not give up and took 0.83 ms per
     // configuration-1 store, the schedule that needs no residency 2.26 ms,
-    // so a give-up is not taken as a sign that the next call would give up
+    // so one give-up is not taken as a sign that the next call would give up
     // too.  `safe_left` counts them down.
     uint32_t safe_after_abort = 0;
     uint32_t safe_left = 0;
-    // The same for calls of long jobs (long_jobs), always: their tiles wait for
-    // every earlier one of the grid's round, so beside a kernel that holds
-    // compute units until all its own workgroups have run, each such launch
-    // gives up, whatever its bound.  Two segments of 32 Mi values beside three
-    // products of 8192 x 8192 matrices: 2630 us a call when every call tries,
-    // 1680 us on average over 65 calls with this (1645 without the one that
-    // tries); on an idle device 107 us, and 149 in the calls after a give-up.
-    uint32_t long_safe_left = 0;
+    // Unless KVSZP_SAFE_CALLS is set: after kGiveUpsInARow persistent encoder
+    // launches of at least `give_up_tiles` tiles gave up one after the other, the
+    // next kTileCalls calls of at least that many run one workgroup per tile
+    // (`tile_calls_left`).  Beside a kernel that holds compute units, whether a
+    // launch gives up follows its length, nearly always or nearly never; see
+    // skip_persistent.
+    bool adapt = true;
+    uint32_t give_ups = 0;
+    uint64_t give_up_tiles = 0;
+    uint32_t tile_calls_left = 0;
     uint64_t safe_calls = 0;      // compress calls run on that schedule
     // Epoch tags run from 1 to epoch_limit, then every tagged word is
     // cleared and they start again (KVSZP_EPOCH_LIMIT lowers the limit so
@@ -302,21 +304,39 @@ int next_epoch(kvszp_ctx* c, hipStream_t stream, uint32_t* epoch) {
     return KVSZP_OK;
 }
 
-constexpr uint32_t kLongSafeCalls = 64;
+// Whether a call whose largest persistent encoder launch would have `tiles`
+// tiles is to run one workgroup per tile, as such launches gave up lately;
+// counted down once per call.  Beside three products of 8192 x 8192 matrices
+// (mean store call, persistent with its give-ups against one workgroup per
+// tile): 1024 blocks of 28 tiles 2960 and 1120 us, 2048 of 56 tiles 3950 and
+// 2340, 40 segments of 250 tiles at odd addresses 2770 and 1240, two of 4096
+// tiles 2630 and 1650, all of which gave up in every call; 357 blocks of 28
+// tiles 925 and 1200, 52 segments of 192 tiles 935 and 1100, which never did.
+// Launches in between give up now and then (256 blocks of 7 and 21 tiles 3 times
+// in 48 calls) and are best left as they are, hence three in a row.
+constexpr uint32_t kGiveUpsInARow = 3;
+constexpr uint32_t kTileCalls = 64;
 
-// True when a call of long jobs is to run without the persistent encoder, as a
-// recent one gave up; counted down once per call.
-bool skip_long_encoder(kvszp_ctx* c, bool long_call) {
-    if (!long_call || c->long_safe_left == 0) return false;
-    c->long_safe_left -= 1;
+bool skip_persistent(kvszp_ctx* c, uint64_t tiles) {
+    if (c->tile_calls_left == 0 || tiles < c->give_up_tiles) return false;
+    c->tile_calls_left -= 1;
     c->safe_calls += 1;
     return true;
 }
 
-// A launch of the call gave up (`long_call`: on the persistent encoder for long jobs).
-void note_give_up(kvszp_ctx* c, bool long_call) {
-    c->safe_left = c->safe_after_abort;
-    if (long_call) c->long_safe_left = kLongSafeCalls;
+// The outcome of a call whose largest persistent encoder launch had `tiles` tiles.
+void note_persistent(kvszp_ctx* c, uint64_t tiles, bool gave_up) {
+    if (!c->adapt) return;
+    if (gave_up) {
+        c->give_up_tiles = c->give_ups == 0 ? tiles : std::min(c->give_up_tiles, tiles);
+        c->give_ups += 1;
+        if (c->give_ups == kGiveUpsInARow) {
+            c->give_ups = 0;
+            c->tile_calls_left = kTileCalls;
+        }
+    } else if (tiles >= c->give_up_tiles) {
+        c->give_ups = 0;
+    }
 }
 
 int check_fixed_config(const kvszp_ctx* c) {
@@ -536,11 +556,19 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
     // needs no residency (pre-pass bound, one workgroup per tile, untimed
     // look-back on earlier workgroups); otherwise the fused bound and the
     // persistent encoder where they apply, with time-bounded waits.
-    bool long_call = false;  // a chunk for the persistent encoder for long jobs
+    auto bound_of = [&](const Chunk& ch, bool safe) -> int {
+        if (!relative) return kBoundAbsolute;
+        return !safe && ch.max_tiles_per_job <= c->fused_tile_limit ? kBoundFused : kBoundPrepass;
+    };
+    auto persistent_takes = [&](const Chunk& ch, bool safe) {
+        return !safe && !f32 &&
+               persistent_encoder_takes(c->pipelined_grid, ch,
+                                        bound_of(ch, safe) == kBoundPrepass, negative_bound);
+    };
+    uint64_t persistent_tiles = 0;  // of the largest persistent launch, or none
     for (const Chunk& ch : chunks)
-        long_call |= !f32 && long_jobs(ch.plain_blocks, ch.max_tiles_per_job) &&
-                     c->pipelined_grid != 0 && !negative_bound;
-    bool skip_long = false;
+        if (persistent_takes(ch, safe)) persistent_tiles = std::max(persistent_tiles, ch.tiles);
+    bool skip = false;              // this call runs one workgroup per tile
     std::vector<char> redo_candidate(chunks.size(), 0);
     std::vector<size_t> chunk_first_job(chunks.size(), 0);
     for (size_t k = 1; k < chunks.size(); ++k) {
@@ -554,16 +582,11 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         std::memset(&p, 0, sizeof(p));
         p.num_groups = fill_groups(p.groups, specs, ch, chunk_first_job[k]);
         p.minmax_shards = minmax_shards(ch.tiles, ch.max_tiles_per_job, batch, kMinMaxWords);
-        int bound_mode = kBoundAbsolute;
-        if (relative)
-            bound_mode = (!safe && ch.max_tiles_per_job <= c->fused_tile_limit)
-                             ? kBoundFused : kBoundPrepass;
+        const int bound_mode = bound_of(ch, safe);
         const bool prepass = bound_mode == kBoundPrepass;
-        const bool lng = long_jobs(ch.plain_blocks, ch.max_tiles_per_job);
-        const bool persistent =
-            !safe && !f32 && !(lng && skip_long) &&
-            persistent_encoder_takes(c->pipelined_grid, ch, prepass, negative_bound);
-        const bool use_arg = persistent && arg_table && !lng;
+        const bool persistent = !skip && persistent_takes(ch, safe);
+        const bool use_arg = persistent && arg_table &&
+                             !long_jobs(ch.plain_blocks, ch.max_tiles_per_job);
         if (!use_arg) {
             const int r = need_table();
             if (r) return r;
@@ -656,7 +679,8 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         c->safe_calls += 1;
         schedule_safe = true;
     }
-    skip_long = skip_long_encoder(c, long_call && !schedule_safe);
+    if (schedule_safe) persistent_tiles = 0;
+    skip = persistent_tiles != 0 && skip_persistent(c, persistent_tiles);
     for (size_t k = 0; k < chunks.size(); ++k)
         if ((rc = launch_chunk(k, schedule_safe, true))) return rc;
 
@@ -664,7 +688,9 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
     // since callers need the sizes on the host (cuszp_wrapper.cpp:520-532).
     hipError_t e = wait_stream(stream);
     if (e != hipSuccess) return hip_fail(e, "waiting for the encoder");
-    if (__atomic_load_n(&c->host_ctl[kHostAbort], __ATOMIC_ACQUIRE) == seq) {
+    const bool gave_up = __atomic_load_n(&c->host_ctl[kHostAbort], __ATOMIC_ACQUIRE) == seq;
+    if (persistent_tiles != 0 && !skip) note_persistent(c, persistent_tiles, gave_up);
+    if (gave_up) {
         // A bounded wait gave up (the device was shared): encode those
         // launches again with the schedule that needs no residency, under
         // fresh epochs.
@@ -673,7 +699,7 @@ int compress_groups(kvszp_ctx* c, const void* const* inputs,
         e = wait_stream(stream);
         if (e != hipSuccess) return hip_fail(e, "waiting for the encoder");
         c->redone += 1;
-        note_give_up(c, long_call);
+        c->safe_left = c->safe_after_abort;
     }
     rc = consume_device_error(c, stream);
     if (rc) return rc;
@@ -936,6 +962,7 @@ int kvszp_create(const kvszp_config* config, int device_id, kvszp_ctx** out) {
         if (const char* sc = std::getenv("KVSZP_SAFE_CALLS")) {
             const long v = std::atol(sc);
             c->safe_after_abort = (uint32_t)std::max(0L, std::min(v, 1L << 20));
+            c->adapt = false;
         }
         if (const char* lim = std::getenv("KVSZP_EPOCH_LIMIT")) {
             const long v = std::atol(lim);
@@ -1233,8 +1260,7 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
     const bool takes = !schedule_safe &&
                        persistent_encoder_takes(c->pipelined_grid, chunk,
                                                 bound_mode == kBoundPrepass, negative_bound);
-    const bool long_call = takes && long_jobs(chunk.plain_blocks, tiles_per_job);
-    const bool persistent = takes && !skip_long_encoder(c, long_call);
+    const bool persistent = takes && !skip_persistent(c, p.total_tiles);
     if (persistent || bound_mode == kBoundFused) {
         p.abort_word = words + kScratchAbort / 8;
         p.wait_ticks = c->wait_ticks;
@@ -1250,7 +1276,8 @@ int kvszp_compress_batch_fixed_bf16_noalloc(
     if (e != hipSuccess) return hip_fail(e, "waiting for the encoder");
     const bool gave_up = p.abort_word != nullptr &&
                          __atomic_load_n(&c->host_ctl[kHostAbort], __ATOMIC_ACQUIRE) == seq;
-    if (gave_up) note_give_up(c, long_call);
+    if (persistent) note_persistent(c, p.total_tiles, gave_up);
+    if (gave_up) c->safe_left = c->safe_after_abort;
     if (p.abort_word != nullptr &&
         (gave_up || __atomic_load_n(&c->host_ctl[kHostOverflow], __ATOMIC_ACQUIRE) == seq)) {
         // Staging overflow, or a bounded wait gave up: the schedule that

@@ -349,8 +349,8 @@ class Context:
 
     def schedule_counts(self) -> dict:
         """Compress calls encoded again (a give-up or a staging overflow)
-        and calls run on the schedule that needs no residency because of a
-        recent give-up."""
+        and calls kept off the persistent encoder because of recent
+        give-ups."""
         r, s = ctypes.c_uint64(), ctypes.c_uint64()
         check(self._lib.kvszp_schedule_counts(self.handle, ctypes.byref(r), ctypes.byref(s)))
         return {"reencoded": r.value, "safe_calls": s.value}

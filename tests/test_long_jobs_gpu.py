@@ -1,7 +1,7 @@
 """The persistent encoder on jobs past the in-kernel exchange (more than 256
 tiles): below and above one round of its grid, a partial last tile, both
-quantizers, relative and absolute bounds, a job whose staging overflows, a
-give-up forced from the host and the calls after it.  Streams and bounds against the oracle."""
+quantizers, relative and absolute bounds, a job whose staging overflows, and
+a give-up forced from the host.  Streams and bounds against the oracle."""
 
 from __future__ import annotations
 
@@ -94,63 +94,3 @@ def test_give_up(oracle):
     w._ctx.set_wait_bound(0)
     pages = pages_of(2, MANY)
     until_give_up(w._ctx, lambda: store_and_check(oracle, w, pages, 1e-4, True, 0))
-
-
-AFTER = 64  # long calls after a give-up that stay off the persistent encoder
-
-
-def test_calls_after_a_give_up(oracle):
-    w = wrapper(True)
-    w._ctx.set_wait_bound(0)
-    pages = pages_of(2, MANY)
-    bufs = [torch.empty(8 * pages.shape[1], dtype=torch.uint8, device="cuda") for _ in range(2)]
-
-    def store():
-        assert w.compress_batch_fixed_bf16(list(pages), bufs, [1e-4] * 2)[0]
-
-    counts = w._ctx.schedule_counts
-    until_give_up(w._ctx, store)
-    assert counts() == {"reencoded": 1, "safe_calls": 0}
-    store_and_check(oracle, w, pages, 1e-4, True, 0)
-    assert counts() == {"reencoded": 1, "safe_calls": 1}
-    store_and_check(oracle, w, pages_of(40, 9 * 8192), 1e-4, True, 0)  # shorter jobs do not count
-    assert counts()["safe_calls"] == 1
-    before = w._ctx.reencode_count()
-    for _ in range(AFTER - 1):
-        store()
-    assert counts() == {"reencoded": before, "safe_calls": AFTER}
-    until_give_up(w._ctx, store)
-    assert counts()["safe_calls"] == AFTER
-
-
-def test_no_allocation_calls_after_a_give_up(oracle):
-    import ctypes
-
-    import kvszp
-
-    n = MANY
-    pages = pages_of(2, n)
-    bufs = [torch.empty(8 * n, dtype=torch.uint8, device="cuda") for _ in range(2)]
-    ctx = kvszp.Context(kvszp.Config(1e-4, 1, kvszp.DIM_1D, kvszp.MODE_FIXED,
-                                     kvszp.TYPE_FLOAT), 0)
-    ctx.set_wait_bound(0)
-    sizes, bounds = (ctypes.c_uint64 * 2)(), (ctypes.c_float * 2)()
-    host = bits(pages)
-    want = [oracle.compress_page(host[i], n, float(oracle.relative_bound(host[i], n, 1e-4)))
-            for i in range(2)]
-
-    def store():
-        for b in bufs:
-            b.fill_(0xAB)
-        kvszp.check(ctx.compress_noalloc(
-            kvszp.ptr_array([p.data_ptr() for p in pages]),
-            kvszp.ptr_array([b.data_ptr() for b in bufs]), kvszp.u64_array([8 * n] * 2), None,
-            2, n, torch.cuda.current_stream().cuda_stream, sizes, bounds))
-        for i in range(2):
-            assert sizes[i] == len(want[i])
-            assert np.array_equal(bufs[i][:sizes[i]].cpu().numpy(), want[i])
-
-    until_give_up(ctx, store)
-    for safe in (1, 2):
-        store()
-        assert ctx.schedule_counts() == {"reencoded": 1, "safe_calls": safe}
